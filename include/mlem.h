@@ -236,7 +236,9 @@ typedef struct mlem_options {
                              mpicsr4mlem.cpp:536-549,589,657)            */
   const char* checkpoint_dir; /* directory of the checkpoint files (NULL = CWD) */
   int verbose;            /* 1: print the reference driver's stdout lines */
-  int use_graph;          /* 1: run iterations from a captured hipGraph   */
+  int use_graph;          /* 1: long runs replay captured hipGraphs of several
+                             iterations (the same results), short ones are
+                             launched directly; 0: direct launches only     */
   double* loglik;         /* optional [iterations]: FP64 Poisson log-likelihood
                              of each iterate's forward projection          */
   double* fwd_total;      /* optional [iterations]: FP64 sum_i f_i         */
@@ -327,7 +329,8 @@ typedef struct mlem_batch_options {
                        (and alone) at creation and live frames are packed
                        into the blocks that minimise the summed measured
                        time, single frames included                       */
-  int use_graph;    /* 1: replay each iteration from a captured hipGraph  */
+  int use_graph;    /* 1: long runs without a stopping frame replay captured
+                       hipGraphs of several iterations; 0: direct launches  */
   int mode;         /* MLEM_MODE_FAST (default): blocks run through the
                        matrix's box tiling (16x16x4-voxel boxes whose slice
                        of a block, or whose voxel sums, stay in one

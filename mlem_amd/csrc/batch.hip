@@ -644,6 +644,32 @@ void enqueue_iteration(mlem_batch* B, hipStream_t s) {
   check_launch("batched iteration launch");
 }
 
+// n iterations. Blocks change whenever a frame stops, and a captured graph
+// with them (0.1-0.4 ms to build), so iterations are launched directly; runs
+// of at least kGraphMin are replayed kGraphIterations at a time.
+constexpr int kGraphIterations = 16, kGraphMin = 96;
+void enqueue_iterations(mlem_batch* B, int n, hipStream_t s) {
+  int i = 0;
+  if (B->use_graph) {
+    if (!B->exec && n >= kGraphMin) {
+      MLEM_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+      try {
+        for (int k = 0; k < kGraphIterations; ++k) enqueue_iteration(B, s);
+      } catch (...) {
+        hipGraph_t g = nullptr;
+        (void)hipStreamEndCapture(s, &g);
+        if (g) (void)hipGraphDestroy(g);
+        throw;
+      }
+      MLEM_HIP(hipStreamEndCapture(s, &B->graph));
+      MLEM_HIP(hipGraphInstantiate(&B->exec, B->graph, nullptr, nullptr, 0));
+    }
+    for (; B->exec && i + kGraphIterations <= n; i += kGraphIterations)
+      MLEM_HIP(hipGraphLaunch(B->exec, s));
+  }
+  for (; i < n; ++i) enqueue_iteration(B, s);
+}
+
 // Measure one block-iteration (forward + backward) at every width on a
 // scratch block (images 1, counts 0, all lanes live); median of 3.
 void tune_widths(mlem_batch* B) {
@@ -913,10 +939,23 @@ int mlem_batch_create(mlem_matrix* h, uint32_t frames, const int32_t* y, uint32_
                             m.stream));
     // x0 per frame: (float)(sum y / sum norm), initImage (seqcsr4mlem.cpp:52-66)
     std::vector<float> x0(frames);
+    std::vector<CountSum> sums(frames, CountSum{0, ~0ull});
+    if ((uint64_t)rows * frames >= kHostSumRows) {
+      struct Buf {
+        CountSum* p = nullptr;
+        ~Buf() { dfree(p); }
+      } d;
+      MLEM_HIP(hipMalloc(&d.p, sizeof(CountSum) * frames));
+      launch_fill(reinterpret_cast<float*>(d.p), 0.f, sizeof(CountSum) / 4 * (size_t)frames,
+                  m.stream);
+      launch_count_sums(B->y_file, rows, frames, d.p, m.stream);
+      MLEM_HIP(hipMemcpyAsync(sums.data(), d.p, sizeof(CountSum) * frames, hipMemcpyDeviceToHost,
+                              m.stream));
+      MLEM_HIP(hipStreamSynchronize(m.stream));
+    }
     for (uint32_t f = 0; f < frames; ++f) {
-      double s = 0.0;
-      const int32_t* yf = y + (size_t)f * rows;
-      for (uint32_t i = 0; i < rows; ++i) s += yf[i];
+      const double s =
+          sums[f].exact() ? (double)sums[f].sum : host_count_sum(y + (size_t)f * rows, rows);
       x0[f] = (float)(s / m.sumnorm);
       hipLaunchKernelGGL(k_lane_fill, dim3(blocks_for(m.cols)), dim3(kBlock), 0, m.stream,
                          B->final_x + (size_t)f * m.cols, 1, 0, x0[f], m.cols);
@@ -970,57 +1009,61 @@ int mlem_batch_run(mlem_batch* B, int max_iterations, int* iterations_run) {
       B->graph_gen = m.launch_gen;
     }
     int it = 0;
-    for (; it < max_iterations && !B->blocks.empty(); ++it) {
-      if (B->use_graph) {
-        if (!B->exec) {
-          MLEM_HIP(hipStreamBeginCapture(m.stream, hipStreamCaptureModeThreadLocal));
-          try {
-            enqueue_iteration(B, m.stream);
-          } catch (...) {
-            hipGraph_t g = nullptr;
-            (void)hipStreamEndCapture(m.stream, &g);
-            if (g) (void)hipGraphDestroy(g);
-            throw;
-          }
-          MLEM_HIP(hipStreamEndCapture(m.stream, &B->graph));
-          MLEM_HIP(hipGraphInstantiate(&B->exec, B->graph, nullptr, nullptr, 0));
-        }
-        MLEM_HIP(hipGraphLaunch(B->exec, m.stream));
-      } else {
-        enqueue_iteration(B, m.stream);
+    while (it < max_iterations && !B->blocks.empty()) {
+      // Iterations until a frame can stop: with budgets alone, the blocks
+      // stay as they are until the smallest remaining budget is spent, so
+      // the host need not wait for every iteration's statistics.
+      int n = 1;
+      if (B->tol <= 0.0) {
+        n = std::min(max_iterations - it, (int)kRing);
+        for (uint32_t f = 0; f < B->F; ++f)
+          if (B->active[f]) n = std::min(n, B->budget[f] - B->done[f]);
+        n = std::max(n, 1);
       }
-      // per-frame statistics of this iteration
+      enqueue_iterations(B, n, m.stream);
+      // per-frame statistics of these iterations: each block's ring slots
+      // (all of them when they wrap around)
       bool changed = false;
       std::vector<std::vector<double2>> res(B->blocks.size());
+      std::vector<unsigned> first(B->blocks.size());
       for (size_t i = 0; i < B->blocks.size(); ++i) {
         const RhsBlock& b = *B->blocks[i];
-        res[i].resize((size_t)b.W);
-        MLEM_HIP(hipMemcpyAsync(res[i].data(), b.results + (size_t)(b.iters % kRing) * b.W,
-                                sizeof(double2) * b.W, hipMemcpyDeviceToHost, m.stream));
+        unsigned lo = b.iters % kRing, cnt = (unsigned)n;
+        if (lo + cnt > kRing) {
+          lo = 0;
+          cnt = kRing;
+        }
+        first[i] = lo;
+        res[i].resize((size_t)cnt * b.W);
+        MLEM_HIP(hipMemcpyAsync(res[i].data(), b.results + (size_t)lo * b.W,
+                                sizeof(double2) * res[i].size(), hipMemcpyDeviceToHost, m.stream));
       }
       MLEM_HIP(hipStreamSynchronize(m.stream));
       for (size_t i = 0; i < B->blocks.size(); ++i) {
         auto& b = B->blocks[i];
-        const std::vector<double2>& r = res[i];
-        b->iters++;
-        for (int l = 0; l < b->W; ++l) {
-          const int f = b->frames[l];
-          if (f < 0 || !B->active[f]) continue;
-          B->done[f]++;
-          B->frame_iterations++;
-          B->ll[f].push_back(r[l].x);
-          const int k = B->done[f];
-          bool stop = k >= B->budget[f];
-          if (!stop && B->tol > 0.0 && k >= 2) {
-            const double a = B->ll[f][k - 1], p = B->ll[f][k - 2];
-            stop = std::fabs(a - p) <= B->tol * std::fabs(a);
-          }
-          if (stop) {
-            B->active[f] = 0;
-            changed = true;
+        for (int k = 0; k < n; ++k) {
+          const double2* r = res[i].data() + (size_t)(b->iters % kRing - first[i]) * b->W;
+          b->iters++;
+          for (int l = 0; l < b->W; ++l) {
+            const int f = b->frames[l];
+            if (f < 0 || !B->active[f]) continue;
+            B->done[f]++;
+            B->frame_iterations++;
+            B->ll[f].push_back(r[l].x);
+            const int d = B->done[f];
+            bool stop = d >= B->budget[f];
+            if (!stop && B->tol > 0.0 && d >= 2) {
+              const double a = B->ll[f][d - 1], p = B->ll[f][d - 2];
+              stop = std::fabs(a - p) <= B->tol * std::fabs(a);
+            }
+            if (stop) {  // only at the last of the n iterations
+              B->active[f] = 0;
+              changed = true;
+            }
           }
         }
       }
+      it += n;
       if (changed) repack(B);
     }
     if (iterations_run) *iterations_run = it;

@@ -357,6 +357,26 @@ template <class T>
 void rows_to_device(const DevMatrix& m, const T* file_order, T* dev, hipStream_t s);
 template <class T>
 void rows_to_file(const DevMatrix& m, const T* dev, T* file_order, hipStream_t s);
+// Sums of int32 counts: sum and sum of magnitudes. While the latter stays
+// below 2^53, every partial sum of the reference's running double sum
+// (seqcsr4mlem.cpp:57-58) is an integer that a double holds exactly, so the
+// integer sum in any order equals it; otherwise the host adds in order.
+struct CountSum {
+  long long sum;
+  unsigned long long magnitude;
+  bool exact() const { return magnitude < (1ull << 53); }
+};
+inline double host_count_sum(const int32_t* y, uint32_t rows) {
+  double s = 0.0;
+  for (uint32_t i = 0; i < rows; ++i) s += y[i];
+  return s;
+}
+// Below this many counts the host's running sum (0.8 ns a count) costs less
+// than the kernel and the read-back of its result (about 25 us).
+constexpr uint32_t kHostSumRows = 32768;
+// out[f] += the sums of y[f*rows .. (f+1)*rows) (out zeroed before).
+void launch_count_sums(const int32_t* y, uint32_t rows, uint32_t frames, CountSum* out,
+                       hipStream_t s);
 // Count column indices >= cols in the CSR (validation).
 void launch_check_columns(const DevMatrix& m, unsigned* bad, hipStream_t s);
 // Build rowptr (u32) from the csr4 END-offset row index already on device.
