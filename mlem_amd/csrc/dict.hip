@@ -1,0 +1,334 @@
+// dict.hip — load-time construction of the dictionary tiles (kernels.hip runs
+// the projections over them), gfx950.
+//
+// Every tile of at most T elements gets the sorted distinct indices it
+// gathers, and every element its 16-bit position among them. The tile's
+// indices are marked in a bitmap in LDS, one slab of 2^18 indices at a time;
+// a prefix sum of the words' population counts gives every marked index its
+// rank, which is its position. Slabs without an element are skipped.
+//
+// What bounds it: the LDS passes over the slabs (clear, mark, count, look up;
+// about 1 us each for a 1024-lane workgroup, two of them per CU), 3 slabs per
+// forward tile of the 128x128x48 matrix and 6 per backward tile. It replaces a
+// bitonic sort of 8-byte keys in LDS (105 passes over a 128 KB array): both
+// projections' two passes 129 -> 4.9 ms on that matrix (168.5M elements), 600 ->
+// 40 ms on the 192x192x64 one (789.8M, 9 and 16 slabs). The sort would be
+// faster only where a tile's indices spread over more than about 800 slabs,
+// 2 * 10^8 rows or columns.
+#include <algorithm>
+#include <vector>
+
+#include "internal.hpp"
+#include "mlem.h"
+
+namespace mlem {
+namespace {
+
+constexpr int kBlock = 256;
+constexpr uint32_t kWave = 64;
+constexpr uint32_t kBuild = 1024;                 // lanes of a build workgroup
+constexpr uint32_t kSlabBits = 18;                // indices per bitmap slab (log2)
+constexpr uint32_t kWords = (1u << kSlabBits) / 32;
+constexpr uint32_t kLaneWords = kWords / kBuild;  // words counted by one lane
+constexpr uint32_t kMaxSlabs = 1u << (32 - kSlabBits);
+static_assert(kLaneWords == 8, "word() pads every lane's run of 8 words");
+
+// Word w of the bitmap: one word of padding after every 8, so that the lanes'
+// runs of 8 words start in different LDS banks.
+__device__ __forceinline__ uint32_t word(uint32_t w) { return w + (w >> 3); }
+
+void check_launch(const char* what) {
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) raise(MLEM_EDEVICE, std::string(what) + ": " + hipGetErrorString(e));
+}
+
+// One tile per workgroup, at most EB elements per lane. Pass 1 (tiles4 ==
+// nullptr) counts the distinct indices of every tile; pass 2 writes the
+// dictionary, padded with zeros to whole rounds of `nb` entries, and the
+// {value, position} element arrays, padded with zeros to 64 elements. Indices
+// are below slab_words * 32 * 2^18.
+template <uint32_t EB, int VK>
+__global__ __launch_bounds__(kBuild) void k_dict_rank(const uint2* __restrict__ el,
+                                                      const uint2* __restrict__ tiles2,
+                                                      const uint4* __restrict__ tiles4,
+                                                      uint32_t nb, uint32_t slab_words,
+                                                      uint32_t* __restrict__ nd_out,
+                                                      uint32_t* __restrict__ dict,
+                                                      void* __restrict__ dval,
+                                                      uint16_t* __restrict__ dlix) {
+  constexpr uint32_t T = kBuild * EB;
+  __shared__ uint32_t bits[kWords + kWords / 8];
+  __shared__ uint16_t before[kWords + kWords / 8];  // marked indices before each word
+  __shared__ uint32_t slabs[kMaxSlabs / 32];        // slabs that hold an element
+  __shared__ uint32_t wsum[kBuild / kWave + 1];
+  const uint32_t tile = blockIdx.x, t = threadIdx.x, lane = t % kWave, wave = t / kWave;
+  uint32_t e0, e1, a0 = 0, g0 = 0;
+  if (tiles4) {
+    const uint4 a = tiles4[tile], b = tiles4[tile + 1];
+    e0 = a.y;
+    e1 = b.y;
+    a0 = a.z;
+    g0 = a.w;
+  } else {
+    e0 = tiles2[tile].y;
+    e1 = tiles2[tile + 1].y;
+  }
+  const uint32_t count = e1 - e0;
+  if (count > T || count == 0) {  // one long segment, or nothing: no dictionary
+    if (!tiles4 && t == 0) nd_out[tile] = 0;
+    return;
+  }
+  uint2 e[EB];
+  uint32_t pos[EB];
+#pragma unroll
+  for (uint32_t j = 0; j < EB; ++j) e[j] = el[e0 + min(t + j * kBuild, count - 1)];
+  if (t < kMaxSlabs / 32) slabs[t] = 0;
+  __syncthreads();
+#pragma unroll
+  for (uint32_t j = 0; j < EB; ++j) {
+    pos[j] = 0;
+    const uint32_t s = e[j].x >> kSlabBits;
+    if (!((slabs[s >> 5] >> (s & 31u)) & 1u)) atomicOr(&slabs[s >> 5], 1u << (s & 31u));
+  }
+  __syncthreads();
+  uint32_t total = 0;  // distinct indices in the slabs so far (uniform)
+  for (uint32_t sw = 0; sw < slab_words; ++sw) {
+    for (uint32_t left = slabs[sw]; left; left &= left - 1) {  // uniform
+      const uint32_t s = sw * 32 + (uint32_t)__builtin_ctz(left);
+      for (uint32_t w = t; w < kWords + kWords / 8; w += kBuild) bits[w] = 0;
+      __syncthreads();
+#pragma unroll
+      for (uint32_t j = 0; j < EB; ++j)
+        if (e[j].x >> kSlabBits == s)
+          atomicOr(&bits[word((e[j].x & ((1u << kSlabBits) - 1)) >> 5)], 1u << (e[j].x & 31u));
+      __syncthreads();
+      uint32_t mine = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < kLaneWords; ++k) mine += __popc(bits[word(t * kLaneWords + k)]);
+      uint32_t run = mine;  // inclusive sum over the wave
+#pragma unroll
+      for (uint32_t d = 1; d < kWave; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)run, d);
+        if (lane >= d) run += o;
+      }
+      if (lane == kWave - 1) wsum[wave] = run;
+      __syncthreads();
+      uint32_t base = total, all = 0;
+      for (uint32_t w = 0; w < kBuild / kWave; ++w) {
+        const uint32_t v = wsum[w];
+        if (w < wave) base += v;
+        all += v;
+      }
+      uint32_t at = base + run - mine;
+#pragma unroll
+      for (uint32_t k = 0; k < kLaneWords; ++k) {
+        const uint32_t w = word(t * kLaneWords + k);
+        before[w] = (uint16_t)at;
+        at += __popc(bits[w]);
+      }
+      total += all;
+      __syncthreads();
+      if (tiles4) {
+#pragma unroll
+        for (uint32_t j = 0; j < EB; ++j)
+          if (e[j].x >> kSlabBits == s) {
+            const uint32_t w = word((e[j].x & ((1u << kSlabBits) - 1)) >> 5), b = e[j].x & 31u;
+            pos[j] = before[w] + __popc(bits[w] & ((1u << b) - 1u));
+            dict[g0 + pos[j]] = e[j].x;  // equal indices write the same word
+          }
+      }
+      __syncthreads();  // the next slab clears the bitmap
+    }
+  }
+  if (!tiles4) {
+    if (t == 0) nd_out[tile] = total;
+    return;
+  }
+  for (uint32_t i = total + t; i < (total + nb - 1) / nb * nb; i += kBuild) dict[g0 + i] = 0;
+  const uint32_t padded = (count + 63) / 64 * 64;
+#pragma unroll
+  for (uint32_t j = 0; j < EB; ++j) {
+    const uint32_t i = t + j * kBuild;
+    if (i >= padded) continue;
+    const bool in = i < count;
+    const uint32_t v = in ? e[j].y : 0u;  // fp32 bits; 16-bit kinds hold exact values
+    dlix[a0 + i] = in ? (uint16_t)pos[j] : (uint16_t)0;
+    if constexpr (VK == kF32)
+      static_cast<uint32_t*>(dval)[a0 + i] = v;
+    else if constexpr (VK == kF16)
+      static_cast<uint16_t*>(dval)[a0 + i] =
+          __builtin_bit_cast(uint16_t, (_Float16)__uint_as_float(v));
+    else
+      static_cast<uint16_t*>(dval)[a0 + i] = (uint16_t)(v >> 16);
+  }
+}
+
+// Packs every 64-entry dictionary slot in place, one wave per slot: when the
+// slot's ascending indices span less than 2^16 they become 16-bit offsets
+// from the first (two per word, in the slot's first 32 words); meta[slot] =
+// first index, with bit 31 set when the slot keeps its 32-bit indices.
+// Unused entries at a tile's end hold 0 (below the first index) and become
+// offset 0.
+__global__ __launch_bounds__(kBlock) void k_dict_pack(uint32_t* __restrict__ dict,
+                                                      uint32_t* __restrict__ meta,
+                                                      uint64_t nslots) {
+  const uint64_t s = (uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+  if (s >= nslots) return;  // whole waves
+  const uint32_t l = threadIdx.x % kWave;
+  const uint32_t v = dict[s * kWave + l];
+  const uint32_t base = __shfl(v, 0);
+  uint32_t hi = v;
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) hi = max(hi, (uint32_t)__shfl_xor(hi, off));
+  const bool wide = hi - base > 0xFFFFu;
+  if (!wide) {
+    const uint32_t o = v >= base ? v - base : 0u;
+    const uint32_t o1 = __shfl_down(o, 1);
+    if ((l & 1) == 0) dict[s * kWave + (l >> 1)] = o | (o1 << 16);
+  }
+  if (l == 0) meta[s] = base | (wide ? 0x80000000u : 0u);
+}
+
+// Build the dictionary format of one projection from its device-order
+// segments (host copy of the pointers, device 8-byte records). The format
+// depends on the tile size T = NB*EPT and the segment limit NB.
+template <int NB, int EPT, int VK>
+void build_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, DictFormat& D,
+                hipStream_t s) {
+  const uint32_t slab_words = (uint32_t)((((uint64_t)dim + (1u << kSlabBits) - 1) >> kSlabBits) + 31) / 32;
+  constexpr uint32_t T = NB * EPT;
+  static_assert(T % kBuild == 0, "build workgroups cover whole tiles");
+  constexpr uint32_t EB = T / kBuild;  // elements per build lane
+  const std::vector<uint32_t> tl = partition_tiles(ptr, T, NB);
+  const uint32_t nt = (uint32_t)tl.size() - 1;
+  std::vector<uint2> d2(tl.size());
+  for (size_t i = 0; i < tl.size(); ++i) d2[i] = make_uint2(tl[i], ptr[tl[i]]);
+  struct Buf {
+    void* p = nullptr;
+    ~Buf() {
+      if (p) (void)hipFree(p);
+    }
+  } t2, ndb;
+  MLEM_HIP(hipMalloc(&t2.p, sizeof(uint2) * d2.size()));
+  MLEM_HIP(hipMalloc(&ndb.p, 4ull * std::max<uint32_t>(nt, 1)));
+  MLEM_HIP(hipMemcpyAsync(t2.p, d2.data(), sizeof(uint2) * d2.size(), hipMemcpyHostToDevice, s));
+  std::vector<uint32_t> nd(nt);
+  if (nt) {
+    hipLaunchKernelGGL((k_dict_rank<EB, VK>), dim3(nt), dim3(kBuild), 0, s, (const uint2*)el,
+                       (const uint2*)t2.p, (const uint4*)nullptr, (uint32_t)NB, slab_words,
+                       (uint32_t*)ndb.p,
+                       (uint32_t*)nullptr, (void*)nullptr, (uint16_t*)nullptr);
+    check_launch("dictionary count launch");
+    MLEM_HIP(hipMemcpyAsync(nd.data(), ndb.p, 4ull * nt, hipMemcpyDeviceToHost, s));
+    MLEM_HIP(hipStreamSynchronize(s));
+  }
+  std::vector<uint4> d4(tl.size());
+  uint64_t acc_a = 0, acc_g = 0;
+  for (uint32_t i = 0; i <= nt; ++i) {
+    d4[i] = make_uint4(tl[i], ptr[tl[i]], (uint32_t)acc_a, (uint32_t)acc_g);
+    if (i == nt) break;
+    const uint32_t count = ptr[tl[i + 1]] - ptr[tl[i]];
+    if (count <= T) acc_a += (count + 63) / 64 * 64;
+    acc_g += (nd[i] + NB - 1) / NB * NB;  // whole rounds of one slot per wave
+  }
+  if (acc_a + T > 0xFFFFFFFFull || acc_g > 0xFFFFFFFFull)
+    raise(MLEM_EINVAL, "matrix too large for the dictionary format");
+  free_dict(D);
+  D.ntiles = nt;
+  D.vk = VK;
+  D.ndict = std::max<uint64_t>(acc_g, NB);
+  D.nval = acc_a + T;  // tail: full-tile loads of the last tile stay in bounds
+  const uint64_t vb = VK == kF32 ? 4 : 2;
+  const uint64_t nslots = D.ndict / kWave;
+  const uint64_t tail = (uint64_t)(NB / kWave) * EPT;  // rounded-up rounds of the last tile
+  MLEM_HIP(hipMalloc(&D.tiles, sizeof(uint4) * d4.size()));
+  MLEM_HIP(hipMalloc(&D.dict, 4ull * D.ndict));
+  MLEM_HIP(hipMalloc(&D.dmeta, 4ull * (nslots + tail)));
+  MLEM_HIP(hipMalloc(&D.dval, vb * D.nval));
+  MLEM_HIP(hipMalloc(&D.dlix, 2ull * D.nval));
+  // the tiles' kernels write everything but what follows the last tile
+  if (acc_g < D.ndict) MLEM_HIP(hipMemsetAsync(D.dict, 0, 4ull * D.ndict, s));
+  MLEM_HIP(hipMemsetAsync(D.dmeta + nslots, 0, 4ull * tail, s));
+  MLEM_HIP(hipMemsetAsync(static_cast<char*>(D.dval) + vb * acc_a, 0, vb * T, s));
+  MLEM_HIP(hipMemsetAsync(D.dlix + acc_a, 0, 2ull * T, s));
+  MLEM_HIP(hipMemcpyAsync(D.tiles, d4.data(), sizeof(uint4) * d4.size(), hipMemcpyHostToDevice, s));
+  if (nt) {
+    hipLaunchKernelGGL((k_dict_rank<EB, VK>), dim3(nt), dim3(kBuild), 0, s, (const uint2*)el,
+                       (const uint2*)nullptr, (const uint4*)D.tiles, (uint32_t)NB, slab_words,
+                       (uint32_t*)nullptr, D.dict, D.dval, D.dlix);
+    check_launch("dictionary fill launch");
+  }
+  const uint64_t per = kBlock / kWave;
+  hipLaunchKernelGGL(k_dict_pack, dim3((unsigned)((nslots + per - 1) / per)), dim3(kBlock), 0, s,
+                     D.dict, D.dmeta, nslots);
+  check_launch("dictionary pack launch");
+  MLEM_HIP(hipStreamSynchronize(s));
+  D.nb = NB;
+  D.ept = EPT;
+}
+
+template <int VK>
+void build_dict_vk(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, int nb, int ept,
+                   DictFormat& D, hipStream_t s) {
+  switch (nb * 1000 + ept) {
+    case 256008: build_dict<256, 8, VK>(ptr, el, dim, D, s); break;
+    case 256016: build_dict<256, 16, VK>(ptr, el, dim, D, s); break;
+    case 256024: build_dict<256, 24, VK>(ptr, el, dim, D, s); break;
+    case 256032: build_dict<256, 32, VK>(ptr, el, dim, D, s); break;
+    case 256048: build_dict<256, 48, VK>(ptr, el, dim, D, s); break;
+    case 256064: build_dict<256, 64, VK>(ptr, el, dim, D, s); break;
+    case 512016: build_dict<512, 16, VK>(ptr, el, dim, D, s); break;
+    case 512024: build_dict<512, 24, VK>(ptr, el, dim, D, s); break;
+    case 512032: build_dict<512, 32, VK>(ptr, el, dim, D, s); break;
+    default: raise(MLEM_EINVAL, "unsupported dictionary tile size");
+  }
+}
+
+}  // namespace
+
+// Greedy partition of segments [0, n) into tiles of at most T elements and
+// `maxseg` segments (one per lane); a segment longer than T forms a tile of
+// its own.
+std::vector<uint32_t> partition_tiles(const std::vector<uint32_t>& ptr, uint32_t T,
+                                      uint32_t maxseg) {
+  const uint32_t n = (uint32_t)ptr.size() - 1;
+  std::vector<uint32_t> tiles{0};
+  uint32_t s = 0;
+  while (s < n) {
+    uint32_t e = s;
+    if (ptr[s + 1] - ptr[s] > T) {
+      e = s + 1;
+    } else {
+      uint64_t cnt = 0;
+      while (e < n && e - s < maxseg && cnt + (ptr[e + 1] - ptr[e]) <= T) {
+        cnt += ptr[e + 1] - ptr[e];
+        ++e;
+      }
+    }
+    tiles.push_back(e);
+    s = e;
+  }
+  return tiles;
+}
+
+void ensure_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, int nb, int ept,
+                 int vk, DictFormat& D, hipStream_t s) {
+  if (D.nb == nb && D.ept == ept && D.vk == vk && D.tiles) return;
+  switch (vk) {
+    case kF32: build_dict_vk<kF32>(ptr, el, dim, nb, ept, D, s); break;
+    case kF16: build_dict_vk<kF16>(ptr, el, dim, nb, ept, D, s); break;
+    case kBF16: build_dict_vk<kBF16>(ptr, el, dim, nb, ept, D, s); break;
+    default: raise(MLEM_EINVAL, "unsupported value storage");
+  }
+}
+
+void free_dict(DictFormat& d) {
+  if (d.tiles) (void)hipFree(d.tiles);
+  if (d.dict) (void)hipFree(d.dict);
+  if (d.dmeta) (void)hipFree(d.dmeta);
+  if (d.dval) (void)hipFree(d.dval);
+  if (d.dlix) (void)hipFree(d.dlix);
+  d = DictFormat();
+}
+
+}  // namespace mlem

@@ -257,6 +257,14 @@ unsigned stats_max_blocks(const DevMatrix& m);
 // layout is built) and (re)build the tile partitions and dictionary formats
 // the launch configuration needs.
 void prepare_tiles(DevMatrix& m, hipStream_t s);
+// Greedy partition of segments [0, n) into tiles of at most T elements and
+// `maxseg` segments: the first segment of every tile, plus n.
+std::vector<uint32_t> partition_tiles(const std::vector<uint32_t>& ptr, uint32_t T,
+                                      uint32_t maxseg);
+// Build a dictionary format (dict.hip) unless D holds it already; `el` indices
+// are below `dim`.
+void ensure_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, int nb, int ept,
+                 int vk, DictFormat& D, hipStream_t s);
 // Release a dictionary format's device memory.
 void free_dict(DictFormat& d);
 // Forward projection. ratio: out = (f != 0) ? y/f : 0, else out = f.

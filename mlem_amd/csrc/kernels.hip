@@ -15,6 +15,7 @@
 //            calcBkProj + calcUpdate, seqcsr4mlem.cpp:108-134). No atomics,
 //            bit-for-bit deterministic.
 //   k_scatter + k_update : the atomic-scatter alternative over the CSR.
+// dict.hip builds the dictionary tiles at load time.
 //
 // G = 1 with EXACT = true gives the reference's rounding sequence: one lane
 // walks a row (column) in ascending order, multiply and add rounded
@@ -809,128 +810,6 @@ __global__ __launch_bounds__(NB) void k_bwd_dict(
   dict_spmv<NB, EPT, VK, EXACT>(colptr, csc, tiles, tile, dval, dlix, dict, dmeta, r, rows, epi);
 }
 
-// Packs every 64-entry dictionary slot in place, one wave per slot: when the
-// slot's ascending indices span less than 2^16 they become 16-bit offsets
-// from the first (two per word, in the slot's first 32 words); meta[slot] =
-// first index, with bit 31 set when the slot keeps its 32-bit indices.
-// Unused entries at a tile's end hold 0 (below the first index) and become
-// offset 0.
-__global__ __launch_bounds__(kBlock) void k_dict_pack(uint32_t* __restrict__ dict,
-                                                      uint32_t* __restrict__ meta,
-                                                      uint64_t nslots) {
-  const uint64_t s = (uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
-  if (s >= nslots) return;  // whole waves
-  const uint32_t l = threadIdx.x % kWave;
-  const uint32_t v = dict[s * kWave + l];
-  const uint32_t base = __shfl(v, 0);
-  uint32_t hi = v;
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) hi = max(hi, (uint32_t)__shfl_xor(hi, off));
-  const bool wide = hi - base > 0xFFFFu;
-  if (!wide) {
-    const uint32_t o = v >= base ? v - base : 0u;
-    const uint32_t o1 = __shfl_down(o, 1);
-    if ((l & 1) == 0) dict[s * kWave + (l >> 1)] = o | (o1 << 16);
-  }
-  if (l == 0) meta[s] = base | (wide ? 0x80000000u : 0u);
-}
-
-constexpr uint32_t pow2_ceil(uint32_t n) {
-  uint32_t p = 1;
-  while (p < n) p <<= 1;
-  return p;
-}
-
-// Dictionary construction, one block per tile. Pass 1 (tiles4 == nullptr)
-// counts the distinct indices of every tile; pass 2 writes the dictionary
-// and the {value, position} element arrays. Keys (index << 16 | element
-// position) are bitonic-sorted in LDS; a block scan of "new index" flags
-// gives every element its dictionary position.
-template <int EPT, int VK>
-__global__ __launch_bounds__(kBlock) void k_dict_build(const uint2* __restrict__ el,
-                                                       const uint2* __restrict__ tiles2,
-                                                       const uint4* __restrict__ tiles4,
-                                                       uint32_t* __restrict__ nd_out,
-                                                       uint32_t* __restrict__ dict,
-                                                       void* __restrict__ dval,
-                                                       uint16_t* __restrict__ dlix) {
-  constexpr uint32_t T = kBlock * EPT;
-  constexpr uint32_t TP = pow2_ceil(T);  // bitonic sort length
-  __shared__ unsigned long long K[TP];
-  __shared__ uint32_t cnt[kBlock + 1];
-  const uint32_t tile = blockIdx.x, t = threadIdx.x;
-  uint32_t e0, e1, a0 = 0, g0 = 0;
-  if (tiles4) {
-    const uint4 a = tiles4[tile], b = tiles4[tile + 1];
-    e0 = a.y;
-    e1 = b.y;
-    a0 = a.z;
-    g0 = a.w;
-  } else {
-    e0 = tiles2[tile].y;
-    e1 = tiles2[tile + 1].y;
-  }
-  const uint32_t count = e1 - e0;
-  if (count > T) {  // one long segment: no dictionary
-    if (!tiles4 && t == 0) nd_out[tile] = 0;
-    return;
-  }
-  for (uint32_t i = t; i < TP; i += kBlock)
-    K[i] = i < count ? (((unsigned long long)el[e0 + i].x << 16) | i) : ~0ull;
-  __syncthreads();
-  for (uint32_t k = 2; k <= TP; k <<= 1) {
-    for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-      for (uint32_t i = t; i < TP; i += kBlock) {
-        const uint32_t ixj = i ^ j;
-        if (ixj > i) {
-          const unsigned long long a = K[i], b = K[ixj];
-          const bool up = (i & k) == 0;
-          if ((a > b) == up) {
-            K[i] = b;
-            K[ixj] = a;
-          }
-        }
-      }
-      __syncthreads();
-    }
-  }
-  // thread t owns sorted entries [t*EPT, t*EPT + EPT)
-  const uint32_t q0 = t * EPT;
-  uint32_t mine = 0;
-  for (uint32_t q = q0; q < q0 + EPT && q < count; ++q)
-    mine += (q == 0 || (K[q] >> 16) != (K[q - 1] >> 16)) ? 1u : 0u;
-  cnt[t] = mine;
-  __syncthreads();
-  if (t == 0) {
-    uint32_t acc = 0;
-    for (int i = 0; i < kBlock; ++i) {
-      const uint32_t c = cnt[i];
-      cnt[i] = acc;
-      acc += c;
-    }
-    cnt[kBlock] = acc;
-  }
-  __syncthreads();
-  if (!tiles4) {
-    if (t == 0) nd_out[tile] = cnt[kBlock];
-    return;
-  }
-  uint32_t rank = cnt[t];
-  for (uint32_t q = q0; q < q0 + EPT && q < count; ++q) {
-    const uint32_t idx = (uint32_t)(K[q] >> 16), pos = (uint32_t)(K[q] & 0xFFFFu);
-    if (q == 0 || (K[q] >> 16) != (K[q - 1] >> 16)) dict[g0 + rank++] = idx;
-    dlix[a0 + pos] = (uint16_t)(rank - 1);
-    const uint32_t bits = el[e0 + pos].y;  // fp32 bits; 16-bit kinds hold exact values
-    if constexpr (VK == kF32)
-      static_cast<uint32_t*>(dval)[a0 + pos] = bits;
-    else if constexpr (VK == kF16)
-      static_cast<uint16_t*>(dval)[a0 + pos] =
-          __builtin_bit_cast(uint16_t, (_Float16)__uint_as_float(bits));
-    else
-      static_cast<uint16_t*>(dval)[a0 + pos] = (uint16_t)(bits >> 16);
-  }
-}
-
 // ------------------------------------------------------ atomic alternative --
 template <int G>
 __global__ __launch_bounds__(kBlock) void k_scatter(const uint32_t* __restrict__ rowptr,
@@ -1301,36 +1180,11 @@ void bwd_d(const DevMatrix& m, const float* r, const float* norm, float* out, bo
   }
 }
 
-// Greedy partition of segments [0, n) into tiles of at most T elements and
-// `maxseg` segments (one per lane); a segment longer than T forms a tile of
-// its own.
-std::vector<uint32_t> partition_tiles(const std::vector<uint32_t>& ptr, uint32_t T,
-                                      uint32_t maxseg = kBlock) {
-  const uint32_t n = (uint32_t)ptr.size() - 1;
-  std::vector<uint32_t> tiles{0};
-  uint32_t s = 0;
-  while (s < n) {
-    uint32_t e = s;
-    if (ptr[s + 1] - ptr[s] > T) {
-      e = s + 1;
-    } else {
-      uint64_t cnt = 0;
-      while (e < n && e - s < maxseg && cnt + (ptr[e + 1] - ptr[e]) <= T) {
-        cnt += ptr[e + 1] - ptr[e];
-        ++e;
-      }
-    }
-    tiles.push_back(e);
-    s = e;
-  }
-  return tiles;
-}
-
 // Tile descriptors {first segment, first element}, ntiles + 1 entries.
 void upload_tiles(const std::vector<uint32_t>& ptr, int ept, uint2*& dev, uint32_t& ntiles,
                   int& cur, hipStream_t s) {
   if (cur == ept && dev) return;
-  const std::vector<uint32_t> t = partition_tiles(ptr, (uint32_t)(kBlock * ept));
+  const std::vector<uint32_t> t = partition_tiles(ptr, (uint32_t)(kBlock * ept), kBlock);
   std::vector<uint2> d(t.size());
   for (size_t i = 0; i < t.size(); ++i) d[i] = make_uint2(t[i], ptr[t[i]]);
   if (dev) (void)hipFree(dev);
@@ -1343,119 +1197,7 @@ void upload_tiles(const std::vector<uint32_t>& ptr, int ept, uint2*& dev, uint32
   cur = ept;
 }
 
-// Build the dictionary format of one projection from its device-order
-// segments (host copy of the pointers, device 8-byte records).
-// The format depends on the tile size T = NB*EPT and the segment limit NB;
-// the build kernel runs 256-lane blocks over the same tiles.
-template <int NB, int EPT, int VK>
-void build_dict(const std::vector<uint32_t>& ptr, const uint2* el, DictFormat& D, hipStream_t s) {
-  constexpr uint32_t T = NB * EPT;
-  static_assert(T % kBlock == 0, "build blocks cover whole tiles");
-  constexpr int EB = T / kBlock;  // elements per build lane
-  const std::vector<uint32_t> tl = partition_tiles(ptr, T, NB);
-  const uint32_t nt = (uint32_t)tl.size() - 1;
-  std::vector<uint2> d2(tl.size());
-  for (size_t i = 0; i < tl.size(); ++i) d2[i] = make_uint2(tl[i], ptr[tl[i]]);
-  struct Buf {
-    void* p = nullptr;
-    ~Buf() {
-      if (p) (void)hipFree(p);
-    }
-  } t2, ndb;
-  MLEM_HIP(hipMalloc(&t2.p, sizeof(uint2) * d2.size()));
-  MLEM_HIP(hipMalloc(&ndb.p, 4ull * std::max<uint32_t>(nt, 1)));
-  MLEM_HIP(hipMemcpyAsync(t2.p, d2.data(), sizeof(uint2) * d2.size(), hipMemcpyHostToDevice, s));
-  std::vector<uint32_t> nd(nt);
-  if (nt) {
-    hipLaunchKernelGGL((k_dict_build<EB, VK>), dim3(nt), dim3(kBlock), 0, s, (const uint2*)el,
-                       (const uint2*)t2.p, (const uint4*)nullptr, (uint32_t*)ndb.p,
-                       (uint32_t*)nullptr, (void*)nullptr, (uint16_t*)nullptr);
-    check_launch("dictionary count launch");
-    MLEM_HIP(hipMemcpyAsync(nd.data(), ndb.p, 4ull * nt, hipMemcpyDeviceToHost, s));
-    MLEM_HIP(hipStreamSynchronize(s));
-  }
-  std::vector<uint4> d4(tl.size());
-  uint64_t acc_a = 0, acc_g = 0;
-  for (uint32_t i = 0; i <= nt; ++i) {
-    d4[i] = make_uint4(tl[i], ptr[tl[i]], (uint32_t)acc_a, (uint32_t)acc_g);
-    if (i == nt) break;
-    const uint32_t count = ptr[tl[i + 1]] - ptr[tl[i]];
-    if (count <= T) acc_a += (count + 63) / 64 * 64;
-    acc_g += (nd[i] + NB - 1) / NB * NB;  // whole rounds of one slot per wave
-  }
-  if (acc_a + T > 0xFFFFFFFFull || acc_g > 0xFFFFFFFFull)
-    raise(MLEM_EINVAL, "matrix too large for the dictionary format");
-  free_dict(D);
-  D.ntiles = nt;
-  D.vk = VK;
-  D.ndict = std::max<uint64_t>(acc_g, NB);
-  D.nval = acc_a + T;  // tail: full-tile loads of the last tile stay in bounds
-  const uint64_t vbytes = (VK == kF32 ? 4ull : 2ull) * D.nval;
-  const uint64_t nslots = D.ndict / kWave;
-  const uint64_t nmeta = nslots + (uint64_t)(NB / kWave) * EPT;  // tail: rounded-up rounds
-  MLEM_HIP(hipMalloc(&D.tiles, sizeof(uint4) * d4.size()));
-  MLEM_HIP(hipMalloc(&D.dict, 4ull * D.ndict));
-  MLEM_HIP(hipMalloc(&D.dmeta, 4ull * nmeta));
-  MLEM_HIP(hipMalloc(&D.dval, vbytes));
-  MLEM_HIP(hipMalloc(&D.dlix, 2ull * D.nval));
-  MLEM_HIP(hipMemsetAsync(D.dict, 0, 4ull * D.ndict, s));
-  MLEM_HIP(hipMemsetAsync(D.dmeta, 0, 4ull * nmeta, s));
-  MLEM_HIP(hipMemsetAsync(D.dval, 0, vbytes, s));
-  MLEM_HIP(hipMemsetAsync(D.dlix, 0, 2ull * D.nval, s));
-  MLEM_HIP(hipMemcpyAsync(D.tiles, d4.data(), sizeof(uint4) * d4.size(), hipMemcpyHostToDevice, s));
-  if (nt) {
-    hipLaunchKernelGGL((k_dict_build<EB, VK>), dim3(nt), dim3(kBlock), 0, s, (const uint2*)el,
-                       (const uint2*)nullptr, (const uint4*)D.tiles, (uint32_t*)nullptr, D.dict,
-                       D.dval, D.dlix);
-    check_launch("dictionary fill launch");
-    const uint64_t per = kBlock / kWave;
-    hipLaunchKernelGGL(k_dict_pack, dim3((unsigned)((nslots + per - 1) / per)), dim3(kBlock), 0, s,
-                       D.dict, D.dmeta, nslots);
-    check_launch("dictionary pack launch");
-  }
-  MLEM_HIP(hipStreamSynchronize(s));
-  D.nb = NB;
-  D.ept = EPT;
-}
-
-template <int VK>
-void build_dict_vk(const std::vector<uint32_t>& ptr, const uint2* el, int nb, int ept,
-                   DictFormat& D, hipStream_t s) {
-  switch (nb * 1000 + ept) {
-    case 256008: build_dict<256, 8, VK>(ptr, el, D, s); break;
-    case 256016: build_dict<256, 16, VK>(ptr, el, D, s); break;
-    case 256024: build_dict<256, 24, VK>(ptr, el, D, s); break;
-    case 256032: build_dict<256, 32, VK>(ptr, el, D, s); break;
-    case 256048: build_dict<256, 48, VK>(ptr, el, D, s); break;
-    case 256064: build_dict<256, 64, VK>(ptr, el, D, s); break;
-    case 512016: build_dict<512, 16, VK>(ptr, el, D, s); break;
-    case 512024: build_dict<512, 24, VK>(ptr, el, D, s); break;
-    case 512032: build_dict<512, 32, VK>(ptr, el, D, s); break;
-    default: raise(MLEM_EINVAL, "unsupported dictionary tile size");
-  }
-}
-
-void ensure_dict(const std::vector<uint32_t>& ptr, const uint2* el, int nb, int ept, int vk,
-                 DictFormat& D, hipStream_t s) {
-  if (D.nb == nb && D.ept == ept && D.vk == vk && D.tiles) return;
-  switch (vk) {
-    case kF32: build_dict_vk<kF32>(ptr, el, nb, ept, D, s); break;
-    case kF16: build_dict_vk<kF16>(ptr, el, nb, ept, D, s); break;
-    case kBF16: build_dict_vk<kBF16>(ptr, el, nb, ept, D, s); break;
-    default: raise(MLEM_EINVAL, "unsupported value storage");
-  }
-}
-
 }  // namespace
-
-void free_dict(DictFormat& d) {
-  if (d.tiles) (void)hipFree(d.tiles);
-  if (d.dict) (void)hipFree(d.dict);
-  if (d.dmeta) (void)hipFree(d.dmeta);
-  if (d.dval) (void)hipFree(d.dval);
-  if (d.dlix) (void)hipFree(d.dlix);
-  d = DictFormat();
-}
 
 void prepare_tiles(DevMatrix& m, hipStream_t s) {
   if (m.h_rowptr.size() != (size_t)m.rows + 1) {
@@ -1475,9 +1217,9 @@ void prepare_tiles(DevMatrix& m, hipStream_t s) {
   if (m.bwd.kind == kTiles && m.csc)
     upload_tiles(m.h_colptr, m.bwd.ept, m.tiles_bwd, m.ntiles_bwd, m.tiles_bwd_ept, s);
   if (is_dict(m.fwd.kind))
-    ensure_dict(m.h_rowptr, m.csr, dict_lanes(m.fwd.kind), m.fwd.ept, m.vk, m.dfwd, s);
+    ensure_dict(m.h_rowptr, m.csr, m.cols, dict_lanes(m.fwd.kind), m.fwd.ept, m.vk, m.dfwd, s);
   if (is_dict(m.bwd.kind) && m.csc)
-    ensure_dict(m.h_colptr, m.csc, dict_lanes(m.bwd.kind), m.bwd.ept, m.vk, m.dbwd, s);
+    ensure_dict(m.h_colptr, m.csc, m.rows, dict_lanes(m.bwd.kind), m.bwd.ept, m.vk, m.dbwd, s);
 }
 
 // Blocks of the statistics-producing forward launch: the larger of the FAST
