@@ -243,6 +243,34 @@ GroupLaunch make_launch(int kind, int param) {
   return g;
 }
 
+// Dictionary tiles of a projection whose segments end at ptr. 16384-element
+// tiles run by 512-lane blocks, two per CU (LDS- and register-bound), are the
+// fastest once every CU gets several: pet (168.4M elements) forward / backward
+// 224 / 218 us against 250 / 246 with 8192. A small matrix is bound by the
+// latency of one tile and by its last wave of tiles (us, 16384 / 8192 / 2048
+// elements, launch included):
+//   29.5M elements  50.3 / 54.2 / 64.1 forward, 44.3 / 45.2 / 60.3 backward
+//   25.4M           41.3 / 41.7 / 44.4,          41.9 / 43.4 / 61.8
+//    9.7M           23.2 / 20.8 / 21.1,          23.0 / 22.2 / 30.2
+//    3.7M           13.2 / 12.2 / 12.2,          13.0 / 11.7 / 12.8
+//    1.9M           12.4 / 10.1 /  9.3,          12.2 /  9.5 /  9.1
+//    0.5M           11.4 /  9.5 /  7.7,          10.7 /  9.0 /  6.9
+// A segment longer than a tile is summed with direct gathers (EXACT: by one
+// lane), so tiles hold the longest segment where the largest ones can.
+// mlem_autotune measures the alternatives on the real matrix.
+GroupLaunch default_launch(uint64_t nnz, const std::vector<uint32_t>& ptr) {
+  uint32_t longest = 0;
+  if (nnz <= 20000000)
+    for (size_t i = 0; i + 1 < ptr.size(); ++i) longest = std::max(longest, ptr[i + 1] - ptr[i]);
+  GroupLaunch g = make_launch(kDictWide, 32);
+  if (nnz <= 2500000 && longest + 3 <= 256 * 8)
+    g = make_launch(kDict, 8);
+  else if (nnz <= 20000000 && longest + 3 <= 512 * 16)
+    g = make_launch(kDictWide, 16);
+  g.nested = g.kind != kDictWide || g.ept != 32;  // the same FAST sums with every tile size
+  return g;
+}
+
 // Candidate FAST-mode configurations of one projection.
 std::vector<GroupLaunch> launch_candidates() {
   std::vector<GroupLaunch> c;
@@ -371,11 +399,9 @@ void finish_open(mlem_matrix* h, unsigned flags) {
   h->norm_seconds = seconds_since(t0);
 
   const double avgRow = m.rows ? (double)m.nnz / m.rows : 1.0;
-  // 16384-element dictionary tiles run by 512-lane blocks, two per CU (LDS-
-  // and register-bound); mlem_autotune measures the alternatives on the real
-  // matrix.
-  m.fwd = make_launch(kDictWide, 32);
-  m.bwd = make_launch(kDictWide, 32);
+  download_pointers(m, m.stream);
+  m.fwd = default_launch(m.nnz, m.h_rowptr);
+  m.bwd = default_launch(m.nnz, m.h_colptr);
   m.scatter = make_launch(kGroups, lanes_for(avgRow));
   prepare_tiles(m, m.stream);
   if (env_int("MLEM_AUTOTUNE", 0) > 0) autotune(m);

@@ -45,7 +45,8 @@ void check_launch(const char* what) {
 // One tile per workgroup, at most EB elements per lane. Pass 1 (tiles4 ==
 // nullptr) counts the distinct indices of every tile; pass 2 writes the
 // dictionary, padded with zeros to whole rounds of `nb` entries, and the
-// {value, position} element arrays, padded with zeros to 64 elements. Indices
+// {value, position} element arrays, with the tile's leading zero elements and
+// padded with zeros to 64 elements. Indices
 // are below slab_words * 32 * 2^18.
 template <uint32_t EB, int VK>
 __global__ __launch_bounds__(kBuild) void k_dict_rank(const uint2* __restrict__ el,
@@ -62,12 +63,13 @@ __global__ __launch_bounds__(kBuild) void k_dict_rank(const uint2* __restrict__ 
   __shared__ uint32_t slabs[kMaxSlabs / 32];        // slabs that hold an element
   __shared__ uint32_t wsum[kBuild / kWave + 1];
   const uint32_t tile = blockIdx.x, t = threadIdx.x, lane = t % kWave, wave = t / kWave;
-  uint32_t e0, e1, a0 = 0, g0 = 0;
+  uint32_t e0, e1, a0 = 0, lead = 0, g0 = 0;
   if (tiles4) {
     const uint4 a = tiles4[tile], b = tiles4[tile + 1];
     e0 = a.y;
     e1 = b.y;
-    a0 = a.z;
+    a0 = a.z & ~63u;
+    lead = a.z & 63u;
     g0 = a.w;
   } else {
     e0 = tiles2[tile].y;
@@ -145,14 +147,8 @@ __global__ __launch_bounds__(kBuild) void k_dict_rank(const uint2* __restrict__ 
     return;
   }
   for (uint32_t i = total + t; i < (total + nb - 1) / nb * nb; i += kBuild) dict[g0 + i] = 0;
-  const uint32_t padded = (count + 63) / 64 * 64;
-#pragma unroll
-  for (uint32_t j = 0; j < EB; ++j) {
-    const uint32_t i = t + j * kBuild;
-    if (i >= padded) continue;
-    const bool in = i < count;
-    const uint32_t v = in ? e[j].y : 0u;  // fp32 bits; 16-bit kinds hold exact values
-    dlix[a0 + i] = in ? (uint16_t)pos[j] : (uint16_t)0;
+  auto put = [&](uint32_t i, uint32_t v, uint32_t p) {  // v: fp32 bits; 16-bit kinds are exact
+    dlix[a0 + i] = (uint16_t)p;
     if constexpr (VK == kF32)
       static_cast<uint32_t*>(dval)[a0 + i] = v;
     else if constexpr (VK == kF16)
@@ -160,7 +156,13 @@ __global__ __launch_bounds__(kBuild) void k_dict_rank(const uint2* __restrict__ 
           __builtin_bit_cast(uint16_t, (_Float16)__uint_as_float(v));
     else
       static_cast<uint16_t*>(dval)[a0 + i] = (uint16_t)(v >> 16);
-  }
+  };
+#pragma unroll
+  for (uint32_t j = 0; j < EB; ++j)
+    if (t + j * kBuild < count) put(lead + t + j * kBuild, e[j].y, pos[j]);
+  const uint32_t end = lead + count, padded = (end + 63) / 64 * 64;
+  if (t < lead) put(t, 0u, 0u);
+  if (end + t < padded) put(end + t, 0u, 0u);
 }
 
 // Packs every 64-entry dictionary slot in place, one wave per slot: when the
@@ -189,18 +191,43 @@ __global__ __launch_bounds__(kBlock) void k_dict_pack(uint32_t* __restrict__ dic
   if (l == 0) meta[s] = base | (wide ? 0x80000000u : 0u);
 }
 
+// Tiles of at most T elements, leading zeros included, and `maxseg` segments
+// inside the tiles of 16384 elements and 512 segments (DictFormat). A larger
+// tile that is one long segment stays whole.
+std::vector<uint32_t> nested_tiles(const std::vector<uint32_t>& ptr, uint32_t T, uint32_t maxseg,
+                                   std::vector<uint32_t>& lead) {
+  const std::vector<uint32_t> big = partition_tiles(ptr, 16384, 512);
+  std::vector<uint32_t> tiles;
+  lead.clear();
+  for (size_t i = 0; i + 1 < big.size(); ++i)
+    for (uint32_t s = big[i]; s < big[i + 1];) {
+      const uint32_t z = (ptr[s] - ptr[big[i]]) & 3u;
+      uint32_t e = s + 1;
+      while (e < big[i + 1] && e - s < maxseg && (uint64_t)z + (ptr[e + 1] - ptr[s]) <= T) ++e;
+      const uint32_t n = ptr[e] - ptr[s];
+      tiles.push_back(s);
+      lead.push_back(n && n <= T ? z : 0);  // only tiles with stored elements
+      s = e;
+    }
+  tiles.push_back((uint32_t)ptr.size() - 1);
+  return tiles;
+}
+
 // Build the dictionary format of one projection from its device-order
 // segments (host copy of the pointers, device 8-byte records). The format
 // depends on the tile size T = NB*EPT and the segment limit NB.
 template <int NB, int EPT, int VK>
-void build_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, DictFormat& D,
-                hipStream_t s) {
+void build_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, bool nested,
+                DictFormat& D, hipStream_t s) {
   const uint32_t slab_words = (uint32_t)((((uint64_t)dim + (1u << kSlabBits) - 1) >> kSlabBits) + 31) / 32;
   constexpr uint32_t T = NB * EPT;
   static_assert(T % kBuild == 0, "build workgroups cover whole tiles");
   constexpr uint32_t EB = T / kBuild;  // elements per build lane
-  const std::vector<uint32_t> tl = partition_tiles(ptr, T, NB);
+  std::vector<uint32_t> lead;  // leading zero elements of every tile
+  const std::vector<uint32_t> tl =
+      nested ? nested_tiles(ptr, T, NB, lead) : partition_tiles(ptr, T, NB);
   const uint32_t nt = (uint32_t)tl.size() - 1;
+  lead.resize(tl.size(), 0);
   std::vector<uint2> d2(tl.size());
   for (size_t i = 0; i < tl.size(); ++i) d2[i] = make_uint2(tl[i], ptr[tl[i]]);
   struct Buf {
@@ -225,10 +252,10 @@ void build_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim,
   std::vector<uint4> d4(tl.size());
   uint64_t acc_a = 0, acc_g = 0;
   for (uint32_t i = 0; i <= nt; ++i) {
-    d4[i] = make_uint4(tl[i], ptr[tl[i]], (uint32_t)acc_a, (uint32_t)acc_g);
+    d4[i] = make_uint4(tl[i], ptr[tl[i]], (uint32_t)acc_a | lead[i], (uint32_t)acc_g);
     if (i == nt) break;
     const uint32_t count = ptr[tl[i + 1]] - ptr[tl[i]];
-    if (count <= T) acc_a += (count + 63) / 64 * 64;
+    if (count <= T) acc_a += (lead[i] + count + 63) / 64 * 64;
     acc_g += (nd[i] + NB - 1) / NB * NB;  // whole rounds of one slot per wave
   }
   if (acc_a + T > 0xFFFFFFFFull || acc_g > 0xFFFFFFFFull)
@@ -265,21 +292,22 @@ void build_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim,
   MLEM_HIP(hipStreamSynchronize(s));
   D.nb = NB;
   D.ept = EPT;
+  D.nested = nested;
 }
 
 template <int VK>
 void build_dict_vk(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, int nb, int ept,
-                   DictFormat& D, hipStream_t s) {
+                   bool nested, DictFormat& D, hipStream_t s) {
   switch (nb * 1000 + ept) {
-    case 256008: build_dict<256, 8, VK>(ptr, el, dim, D, s); break;
-    case 256016: build_dict<256, 16, VK>(ptr, el, dim, D, s); break;
-    case 256024: build_dict<256, 24, VK>(ptr, el, dim, D, s); break;
-    case 256032: build_dict<256, 32, VK>(ptr, el, dim, D, s); break;
-    case 256048: build_dict<256, 48, VK>(ptr, el, dim, D, s); break;
-    case 256064: build_dict<256, 64, VK>(ptr, el, dim, D, s); break;
-    case 512016: build_dict<512, 16, VK>(ptr, el, dim, D, s); break;
-    case 512024: build_dict<512, 24, VK>(ptr, el, dim, D, s); break;
-    case 512032: build_dict<512, 32, VK>(ptr, el, dim, D, s); break;
+    case 256008: build_dict<256, 8, VK>(ptr, el, dim, nested, D, s); break;
+    case 256016: build_dict<256, 16, VK>(ptr, el, dim, nested, D, s); break;
+    case 256024: build_dict<256, 24, VK>(ptr, el, dim, nested, D, s); break;
+    case 256032: build_dict<256, 32, VK>(ptr, el, dim, nested, D, s); break;
+    case 256048: build_dict<256, 48, VK>(ptr, el, dim, nested, D, s); break;
+    case 256064: build_dict<256, 64, VK>(ptr, el, dim, nested, D, s); break;
+    case 512016: build_dict<512, 16, VK>(ptr, el, dim, nested, D, s); break;
+    case 512024: build_dict<512, 24, VK>(ptr, el, dim, nested, D, s); break;
+    case 512032: build_dict<512, 32, VK>(ptr, el, dim, nested, D, s); break;
     default: raise(MLEM_EINVAL, "unsupported dictionary tile size");
   }
 }
@@ -312,12 +340,12 @@ std::vector<uint32_t> partition_tiles(const std::vector<uint32_t>& ptr, uint32_t
 }
 
 void ensure_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, int nb, int ept,
-                 int vk, DictFormat& D, hipStream_t s) {
-  if (D.nb == nb && D.ept == ept && D.vk == vk && D.tiles) return;
+                 bool nested, int vk, DictFormat& D, hipStream_t s) {
+  if (D.nb == nb && D.ept == ept && D.nested == nested && D.vk == vk && D.tiles) return;
   switch (vk) {
-    case kF32: build_dict_vk<kF32>(ptr, el, dim, nb, ept, D, s); break;
-    case kF16: build_dict_vk<kF16>(ptr, el, dim, nb, ept, D, s); break;
-    case kBF16: build_dict_vk<kBF16>(ptr, el, dim, nb, ept, D, s); break;
+    case kF32: build_dict_vk<kF32>(ptr, el, dim, nb, ept, nested, D, s); break;
+    case kF16: build_dict_vk<kF16>(ptr, el, dim, nb, ept, nested, D, s); break;
+    case kBF16: build_dict_vk<kBF16>(ptr, el, dim, nb, ept, nested, D, s); break;
     default: raise(MLEM_EINVAL, "unsupported value storage");
   }
 }

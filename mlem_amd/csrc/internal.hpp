@@ -81,14 +81,20 @@ inline int dict_lanes(int kind) { return kind == kDictWide ? 512 : 256; }
 
 // Dictionary-tile storage of one projection (built on the device at load
 // time for `nb` lanes per block and `ept` elements per lane: tiles of at most
-// nb*ept elements and nb segments; 0 = not built).
+// nb*ept elements and nb segments; 0 = not built). Nested tiles are cut inside
+// the tiles of 16384 elements and 512 segments and start with the 0 to 3 zero
+// elements that give every element the place modulo 4 it has in the larger
+// tile: a segment's sum is taken in aligned quads, so it is the same bit for
+// bit with either tile size.
 struct DictFormat {
   int nb = 0;
   int ept = 0;
   int vk = 0;                 // value storage (ValueKind): fp32, fp16, bf16
   uint32_t ntiles = 0;
-  uint4* tiles = nullptr;     // [ntiles+1] {first segment, first element,
-                              //  aligned element start, first dict word}
+  bool nested = false;        // tiles inside the 16384-element ones (see below)
+  uint4* tiles = nullptr;     // [ntiles+1] {first segment, first element, element
+                              //  start (a multiple of 64) + leading zero elements,
+                              //  first dict word}
   uint32_t* dict = nullptr;   // distinct gather indices, sorted per tile, in
                               //  64-word slots of 64 entries, nb/64 per round
   uint32_t* dmeta = nullptr;  // per slot: first index | 0x80000000 if 32-bit
@@ -106,6 +112,7 @@ struct GroupLaunch {
   int lanes = 16;          // kGroups: lanes per row (or column)
   int ept = 8;             // kTiles: elements per lane, tile = 256*ept elements
   int blocks_per_cu = 0;   // kGroups: 0 = one block per 256/lanes rows
+  bool nested = false;     // dictionary tiles nested in the 16384-element ones
 };
 
 // A matrix kept in pinned host memory and streamed to the device in row
@@ -254,8 +261,10 @@ struct StatsState {
 // Grid size of a statistics-carrying forward launch (partials needed).
 unsigned stats_max_blocks(const DevMatrix& m);
 // Copy the device-order row/column pointers to the host (once, after the
-// layout is built) and (re)build the tile partitions and dictionary formats
-// the launch configuration needs.
+// layout is built).
+void download_pointers(DevMatrix& m, hipStream_t s);
+// (Re)build the tile partitions and dictionary formats the launch
+// configuration needs.
 void prepare_tiles(DevMatrix& m, hipStream_t s);
 // Greedy partition of segments [0, n) into tiles of at most T elements and
 // `maxseg` segments: the first segment of every tile, plus n.
@@ -264,7 +273,7 @@ std::vector<uint32_t> partition_tiles(const std::vector<uint32_t>& ptr, uint32_t
 // Build a dictionary format (dict.hip) unless D holds it already; `el` indices
 // are below `dim`.
 void ensure_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, int nb, int ept,
-                 int vk, DictFormat& D, hipStream_t s);
+                 bool nested, int vk, DictFormat& D, hipStream_t s);
 // Release a dictionary format's device memory.
 void free_dict(DictFormat& d);
 // Forward projection. ratio: out = (f != 0) ? y/f : 0, else out = f.

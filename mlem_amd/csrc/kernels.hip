@@ -695,7 +695,8 @@ __device__ __forceinline__ void dict_spmv(const uint32_t* __restrict__ segptr,
   __shared__ float red[NB / kWave];
   const uint32_t t = threadIdx.x;
   const uint4 d0 = tiles[tile], d1 = tiles[tile + 1];
-  const uint32_t s0 = d0.x, e0 = d0.y, a0 = d0.z, g0 = d0.w;
+  // the tile's elements follow `lead` zero elements at a0 (see DictFormat)
+  const uint32_t s0 = d0.x, e0 = d0.y, a0 = d0.z & ~63u, lead = d0.z & 63u, g0 = d0.w;
   const uint32_t nseg = d1.x - s0, count = d1.y - e0, nwords = d1.w - g0;
   if (t < nseg) epi.prefetch(s0 + t);
   if (count > T) {
@@ -708,7 +709,7 @@ __device__ __forceinline__ void dict_spmv(const uint32_t* __restrict__ segptr,
     return;
   }
   uint32_t send = 0;
-  if (t < nseg) send = segptr[s0 + t + 1] - e0;
+  if (t < nseg) send = segptr[s0 + t + 1] - e0 + lead;
   W val[H];
   L li[H];
   if (count > 0) {  // block-uniform
@@ -728,7 +729,7 @@ __device__ __forceinline__ void dict_spmv(const uint32_t* __restrict__ segptr,
     load_dict_rounds<NB, 4, EPT>(rounds, ds, rv, rval, rlix, t, V, val, li);
   }
   if (t < nseg) S[t + 1] = send;
-  if (t == 0) S[0] = 0;
+  if (t == 0) S[0] = lead;
   __syncthreads();
   // Products of pack j of this lane are elements NP*(t + j*NB) + q, stored as
   // one NP*4-byte run per pack: no bank conflicts for fp32; two lanes per bank
@@ -1199,7 +1200,7 @@ void upload_tiles(const std::vector<uint32_t>& ptr, int ept, uint2*& dev, uint32
 
 }  // namespace
 
-void prepare_tiles(DevMatrix& m, hipStream_t s) {
+void download_pointers(DevMatrix& m, hipStream_t s) {
   if (m.h_rowptr.size() != (size_t)m.rows + 1) {
     m.h_rowptr.resize((size_t)m.rows + 1);
     MLEM_HIP(hipMemcpyAsync(m.h_rowptr.data(), m.rowptr, 4ull * (m.rows + 1ull),
@@ -1212,14 +1213,20 @@ void prepare_tiles(DevMatrix& m, hipStream_t s) {
                             hipMemcpyDeviceToHost, s));
     MLEM_HIP(hipStreamSynchronize(s));
   }
+}
+
+void prepare_tiles(DevMatrix& m, hipStream_t s) {
+  download_pointers(m, s);
   if (m.fwd.kind == kTiles)
     upload_tiles(m.h_rowptr, m.fwd.ept, m.tiles_fwd, m.ntiles_fwd, m.tiles_fwd_ept, s);
   if (m.bwd.kind == kTiles && m.csc)
     upload_tiles(m.h_colptr, m.bwd.ept, m.tiles_bwd, m.ntiles_bwd, m.tiles_bwd_ept, s);
   if (is_dict(m.fwd.kind))
-    ensure_dict(m.h_rowptr, m.csr, m.cols, dict_lanes(m.fwd.kind), m.fwd.ept, m.vk, m.dfwd, s);
+    ensure_dict(m.h_rowptr, m.csr, m.cols, dict_lanes(m.fwd.kind), m.fwd.ept,
+                m.fwd.nested, m.vk, m.dfwd, s);
   if (is_dict(m.bwd.kind) && m.csc)
-    ensure_dict(m.h_colptr, m.csc, m.rows, dict_lanes(m.bwd.kind), m.bwd.ept, m.vk, m.dbwd, s);
+    ensure_dict(m.h_colptr, m.csc, m.rows, dict_lanes(m.bwd.kind), m.bwd.ept,
+                m.bwd.nested, m.vk, m.dbwd, s);
 }
 
 // Blocks of the statistics-producing forward launch: the larger of the FAST

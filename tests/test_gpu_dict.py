@@ -43,3 +43,42 @@ def test_exact_projections_over_slab_edges(rows, cols, family):
         A.set_launch(family, family)
         assert np.array_equal(M.calcFwProj(A, x, mode="exact"), orc.fwproj(rowidx, el, x))
         assert np.array_equal(M.calcBkProj(A, r, mode="exact"), orc.bkproj(rowidx, el, r, cols))
+
+
+# Small matrices take smaller tiles (2048 elements up to 2.5M elements, 8192 up
+# to 20M, 16384 above, or where a segment does not fit): FAST sums are the same
+# bit for bit as with 16384-element tiles, whatever is chosen.
+@pytest.mark.parametrize("rows,cols,per_row,longest,expect", [
+    (300, 40, 3, 0, ("dict", 8)),            # one tile
+    (5000, 700, 8, 0, ("dict", 8)),          # tiles end at their segment limit
+    (9000, 3000, 60, 0, ("dict", 8)),
+    (9000, 3000, 60, 2045, ("dict", 8)),     # the longest row that fits
+    (9000, 3000, 60, 2046, ("dict512", 16)),
+    (9000, 3000, 60, 8190, ("dict512", 32)),
+    (40000, 30000, 80, 0, ("dict512", 16)),
+])
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+def test_default_tiles_keep_the_sums(rows, cols, per_row, longest, expect, precision):
+    rng = np.random.default_rng(rows + longest)
+    n = rng.integers(0, 2 * per_row + 1, rows)
+    n[rows // 3: rows // 3 + 900] = 0
+    if longest:
+        n[rows // 2] = longest
+    rowidx = np.cumsum(n).astype(np.uint64)
+    el = np.zeros(int(rowidx[-1]), M.ELEMENT_DTYPE)
+    el["column"] = rng.integers(0, cols, el.size)
+    el["value"] = rng.random(el.size, dtype=np.float32)
+    x = rng.random(cols, dtype=np.float32)
+    r = rng.random(rows, dtype=np.float32)
+    y = rng.integers(0, 50, rows).astype(np.int32)
+    with M.Csr4Matrix.from_arrays(rows, cols, rowidx, el, precision=precision) as A:
+        assert A.launch()["fwd"] == expect
+        got = [M.calcFwProj(A, x), M.calcBkProj(A, r), *M.mlem(A, y, None, 4, stats=True)]
+        exact = M.mlem(A, y, None, 4, mode="exact")
+        A.set_launch(("dict512", 32), ("dict512", 32))
+        want = [M.calcFwProj(A, x), M.calcBkProj(A, r), *M.mlem(A, y, None, 4, stats=True)]
+        for a, b in zip(got[:3], want[:3]):
+            assert np.array_equal(a, b)
+        for a, b in zip(got[3:], want[3:]):  # FP64 sums over other workgroups
+            np.testing.assert_allclose(a, b, rtol=1e-12)
+        assert np.array_equal(exact, M.mlem(A, y, None, 4, mode="exact"))
