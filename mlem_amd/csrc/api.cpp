@@ -24,6 +24,7 @@
 #include "internal.hpp"
 #include "mlem.h"
 #include "symmetry.hpp"
+#include "transfer.hpp"
 
 using namespace mlem;
 
@@ -86,43 +87,6 @@ template <class T>
 void dfree(T*& p) {
   if (p) (void)hipFree(p);
   p = nullptr;
-}
-
-// Pinned double-buffered host->device streaming of a large byte range. The
-// producer fills a pinned chunk (file read or memcpy); the copy engine drains
-// it while the next chunk is produced.
-template <class Produce>
-void stream_to_device(void* dst, uint64_t bytes, hipStream_t s, Produce&& produce) {
-  if (bytes == 0) return;
-  const uint64_t kChunk = 64ull << 20;
-  void* pin[2] = {nullptr, nullptr};
-  hipEvent_t ev[2] = {nullptr, nullptr};
-  struct Cleanup {
-    void** pin;
-    hipEvent_t* ev;
-    ~Cleanup() {
-      for (int i = 0; i < 2; ++i) {
-        if (ev[i]) (void)hipEventDestroy(ev[i]);
-        if (pin[i]) (void)hipHostFree(pin[i]);
-      }
-    }
-  } cleanup{pin, ev};
-  for (int i = 0; i < 2; ++i) {
-    MLEM_HIP(hipHostMalloc(&pin[i], kChunk, hipHostMallocDefault));
-    MLEM_HIP(hipEventCreateWithFlags(&ev[i], hipEventDisableTiming));
-  }
-  bool used[2] = {false, false};
-  char* d = static_cast<char*>(dst);
-  for (uint64_t off = 0, i = 0; off < bytes; off += kChunk, ++i) {
-    const int b = (int)(i & 1);
-    const uint64_t n = std::min(kChunk, bytes - off);
-    if (used[b]) MLEM_HIP(hipEventSynchronize(ev[b]));
-    produce(pin[b], off, n);
-    MLEM_HIP(hipMemcpyAsync(d + off, pin[b], n, hipMemcpyHostToDevice, s));
-    MLEM_HIP(hipEventRecord(ev[b], s));
-    used[b] = true;
-  }
-  MLEM_HIP(hipStreamSynchronize(s));
 }
 
 }  // namespace
@@ -710,13 +674,13 @@ int mlem_open(const char* path, unsigned flags, mlem_matrix** out) {
       h.reset(new_matrix(hd.nRows, hd.nColumns, xel.size()));
       upload_rowidx(h->m, xrow.data());
       const char* src = reinterpret_cast<const char*>(xel.data());
-      stream_to_device(h->m.csr, 8ull * xel.size(), h->m.stream,
+      stream_to_device(h->m.csr, 8ull * xel.size(), h->m.device, h->m.stream,
                        [&](void* dst, uint64_t off, uint64_t n) { std::memcpy(dst, src + off, n); });
       h->m.symflags = 0;  // the matrix in HBM is complete
     } else {
       h.reset(new_matrix(hd.nRows, hd.nColumns, hd.nnz));
       upload_rowidx(h->m, rowidx.data());
-      stream_to_device(h->m.csr, 8ull * hd.nnz, h->m.stream, read_at);
+      stream_to_device(h->m.csr, 8ull * hd.nnz, h->m.device, h->m.stream, read_at);
       h->m.symflags = hd.flags & 7u;
     }
     h->m.grid[0] = hd.scanner.grid[0];
@@ -792,7 +756,7 @@ int mlem_open_host(uint32_t rows, uint32_t cols, uint64_t nnz, const uint64_t* r
       for (int k = 0; k < 3; ++k) h->m.grid[k] = grid[k];
     upload_rowidx(h->m, rowidx);
     const char* src = static_cast<const char*>(elements);
-    stream_to_device(h->m.csr, 8ull * nnz, h->m.stream,
+    stream_to_device(h->m.csr, 8ull * nnz, h->m.device, h->m.stream,
                      [&](void* dst, uint64_t off, uint64_t n) { std::memcpy(dst, src + off, n); });
     h->load_seconds = seconds_since(t0);
     finish_open(h.get(), flags);

@@ -80,3 +80,27 @@ def test_count_sums(rows):
         B = M.Batch(A, np.stack([y, y // 2]), [0, 0], block_width=4)
         assert np.array_equal(B.image(0), want)
         assert np.array_equal(B.image(1), orc.init_image(norm, y // 2)[0])
+
+
+# matrices loaded by one thread and by several (from 16 MB on), of less than a
+# chunk (2 MB), whole chunks and with a remainder
+@pytest.mark.parametrize("rows,cols,per_row", [(4095, 4097, 3), (131072, 4096, 2), (131073, 5000, 2),
+                                               (32768, 131071, 64), (33333, 131071, 75)])
+def test_matrices_arrive_whole(rows, cols, per_row):
+    rng = np.random.default_rng(rows)
+    rowidx = np.arange(1, rows + 1, dtype=np.uint64) * per_row
+    el = np.zeros(rows * per_row, M.ELEMENT_DTYPE)
+    el["column"] = rng.integers(0, cols, el.size)
+    el["value"] = rng.random(el.size, dtype=np.float32)
+    x, r = rng.random(cols, dtype=np.float32), rng.random(rows, dtype=np.float32)
+    y = rng.integers(0, 99, rows).astype(np.int32)
+    with M.Csr4Matrix.from_arrays(rows, cols, rowidx, el) as A:
+        norm = M.calcColumnSums(A)
+        assert np.array_equal(norm, orc.column_sums(rowidx, el, cols))
+        assert np.array_equal(M.calcFwProj(A, x, mode="exact"), orc.fwproj(rowidx, el, x))
+        assert np.array_equal(M.calcBkProj(A, r, mode="exact"), orc.bkproj(rowidx, el, r, cols))
+        assert np.array_equal(M.calcCorrel(A, r, y), orc.correl(r, y))
+        u = x.copy()
+        assert np.array_equal(M.calcUpdate(A, norm, norm, u), orc.update(norm, norm, x))
+        assert np.array_equal(M.mlem(A, y, x.copy(), 2, mode="exact", x0_given=True),
+                              orc.mlem(rowidx, el, cols, y, 2, x0=x)[0])
