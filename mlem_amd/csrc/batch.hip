@@ -242,8 +242,7 @@ __device__ __forceinline__ void stat1(int32_t y, float f, double& ll, double& to
 }
 
 // Epilogue of the tiled forward product (FAST mode): a row's piece sums
-// added in box order (read through rowpiece where the forward writes them
-// box by box), then ratio r = (f != 0) ? y/f : 0 and the frames'
+// added in box order, then ratio r = (f != 0) ? y/f : 0 and the frames'
 // FP64 statistics (row groups g, g + groups, ...); one partial per workgroup
 // and frame.
 // (64 VGPRs: the grid of 8 workgroups per CU is resident at once)
@@ -255,24 +254,27 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
                                                         float* __restrict__ R, uint32_t rows,
                                                         double2* __restrict__ partials) {
   constexpr uint32_t L = Quads<W>::L, G = Quads<W>::G;
-  constexpr bool kByBox = panel_slots_by_box(W);  // slots gathered through rowpiece
   const uint32_t q = threadIdx.x % L, g = threadIdx.x / L;
   const uint32_t stride = gridDim.x * G;
   const float4* __restrict__ p4 = reinterpret_cast<const float4*>(part);
   const int4* __restrict__ y4 = reinterpret_cast<const int4*>(Y);
   float4* __restrict__ r4 = reinterpret_cast<float4*>(R);
-  auto slot = [&](uint32_t k) { return kByBox ? rowpiece[k] : k; };
   double ll[4] = {0.0, 0.0, 0.0, 0.0}, tot[4] = {0.0, 0.0, 0.0, 0.0};
   for (uint32_t row = blockIdx.x * G + g; row < rows; row += stride) {
     uint32_t s = rowslot[row];
     const uint32_t e = rowslot[row + 1];
     float4 F = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (; s + 2 <= e; s += 2) {
-      const float4 a0 = p4[(size_t)slot(s) * L + q], a1 = p4[(size_t)slot(s + 1) * L + q];
+    for (; s + 4 <= e; s += 4) {
+      const uint32_t i0 = rowpiece[s], i1 = rowpiece[s + 1], i2 = rowpiece[s + 2],
+                     i3 = rowpiece[s + 3];
+      const float4 a0 = p4[(size_t)i0 * L + q], a1 = p4[(size_t)i1 * L + q];
+      const float4 a2 = p4[(size_t)i2 * L + q], a3 = p4[(size_t)i3 * L + q];
       add4(F, a0);
       add4(F, a1);
+      add4(F, a2);
+      add4(F, a3);
     }
-    if (s < e) add4(F, p4[(size_t)slot(s) * L + q]);
+    for (; s < e; ++s) add4(F, p4[(size_t)rowpiece[s] * L + q]);
     const size_t i = (size_t)row * L + q;
     const int4 y = y4[i];
     r4[i] = make_float4(ratio1(y.x, F.x), ratio1(y.y, F.y), ratio1(y.z, F.z), ratio1(y.w, F.w));
@@ -563,13 +565,13 @@ void launch_tiled_block(mlem_batch* B, RhsBlock& b, hipStream_t s, int set) {
   const PanelFormat& P = *B->P;
   float* fpart = set ? B->fpart2 : B->fpart;
   float* upart = set ? B->upart2 : B->upart;
-  launch_panel_fwd<W>(P, b.X, fpart, B->grid, s);
+  launch_panel_fwd<W>(P, b.X, fpart, s);
   hipLaunchKernelGGL((k_tiled_ratio<W>), dim3(B->grid), dim3(kBlock), 0, s, P.rowslot,
                      P.rowpiece, fpart,
                      b.Y, b.R, m.rows, b.partials);
   hipLaunchKernelGGL((k_batch_stats_reduce<W>), dim3(1), dim3(kReduceLanes), 0, s, b.partials,
                      B->grid, b.counter, b.results, kRing);
-  launch_panel_bwd<W>(P, b.R, upart, B->grid, s);
+  launch_panel_bwd<W>(P, b.R, upart, s);
   hipLaunchKernelGGL((k_tiled_update<W>), dim3(B->grid), dim3(kBlock), 0, s, P.colslot, upart,
                      P.norm, b.X, b.mask, m.cols);
 }
@@ -909,10 +911,10 @@ int mlem_batch_create(mlem_matrix* h, uint32_t frames, const int32_t* y, uint32_
       // the tiling (built once per matrix) and one block's partial sums
       B->P = &ensure_panels(m);
       MLEM_HIP(hipMalloc(&B->fpart, 4ull * std::max<uint64_t>(B->P->nseg, 1) * B->wmax));
-      MLEM_HIP(hipMalloc(&B->upart, 4ull * std::max<uint64_t>(B->P->ngroups, 1) * B->wmax));
+      MLEM_HIP(hipMalloc(&B->upart, 4ull * std::max<uint64_t>(m.cols, 1) * B->wmax));
       if (frames >= 8) {  // room for two tiled blocks: a second stream
         MLEM_HIP(hipMalloc(&B->fpart2, 4ull * std::max<uint64_t>(B->P->nseg, 1) * B->wmax));
-        MLEM_HIP(hipMalloc(&B->upart2, 4ull * std::max<uint64_t>(B->P->ngroups, 1) * B->wmax));
+        MLEM_HIP(hipMalloc(&B->upart2, 4ull * std::max<uint64_t>(m.cols, 1) * B->wmax));
         MLEM_HIP(hipStreamCreateWithFlags(&B->side, hipStreamNonBlocking));
         MLEM_HIP(hipEventCreateWithFlags(&B->fork, hipEventDisableTiming));
         MLEM_HIP(hipEventCreateWithFlags(&B->join, hipEventDisableTiming));

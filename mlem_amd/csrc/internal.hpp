@@ -154,32 +154,38 @@ struct StreamedMatrix {
 // Two-dimensional tiling of the matrix for products with W interleaved
 // right-hand sides (panels.hpp; built on first use by ensure_panels). Vectors
 // of those products index columns in panel order.
+//
+// The forward kernel reads the elements in octets: 8 pieces of a chunk, of about
+// the same length, their elements in quads of 8 x 4: value and column of element
+// 4j + k of piece i at (quad j) * 32 + 4i + k, so that the lanes of a wave load
+// contiguous runs whatever W is. Positions past a piece's end hold value 0 and
+// column kBoxVox, the row of zeros that the kernel keeps in LDS; the last two
+// quads of the arrays hold only those.
 struct PanelFormat {
   uint32_t rows = 0, cols = 0;
-  uint32_t npanels = 0, nchunks = 0;   // boxes, backward chunks
-  uint32_t nfchunks = 0;               // forward chunks
-  uint64_t nseg = 0, ngroups = 0;      // forward slots (pieces), backward slots (voxels)
+  uint32_t npanels = 0;                // boxes
+  uint64_t nseg = 0;                   // pieces, one slot of partial sums each
   uint32_t* pc_of_file = nullptr;      // [cols] panel-order column of each file column
   uint32_t* pc_of_dev = nullptr;       // [cols] ... of each device column
   uint32_t* dev_of_pc = nullptr;       // [cols] device column of each panel-order column
   float* norm = nullptr;               // [cols] column sums in panel order
   uint32_t* pstart = nullptr;          // [npanels+1] first panel-order column of each box
   uint32_t* border = nullptr;          // [npanels] launch order (largest box first)
-  uint32_t* pseg = nullptr;            // [npanels+1] first piece of each box
-  uint32_t* fseg = nullptr;            // [nseg+1] first element of each piece (forward order)
-  uint32_t* fslot = nullptr;           // [nseg] row-major slot of each piece
-  float* fval = nullptr;               // [nnz]
-  uint16_t* fcol = nullptr;            // [nnz] column inside the box
-  uint32_t* rowslot = nullptr;         // [rows+1] first slot of each device row
-  uint32_t* rowpiece = nullptr;        // [nseg] forward-order piece of each row-major slot
+  uint32_t* rowslot = nullptr;         // [rows+1] first entry of each device row in rowpiece
+  uint32_t* rowpiece = nullptr;        // [nseg] the rows' pieces (slots), box order
   uint32_t* pfchunk = nullptr;         // [npanels+1] first forward chunk of each box
-  uint2* fchunk = nullptr;             // [nfchunks+1] {first piece, first element}
+  uint32_t* cpiece = nullptr;          // [chunks+1] first piece of each forward chunk
+  uint32_t* fquad = nullptr;           // [chunks*128+1] first quad of each octet
+  uint32_t* fpiece = nullptr;          // [chunks*1024] slot of each piece, ~0: none
+  float* fval = nullptr;               // [quads+2][8][4]
+  uint16_t* fcol = nullptr;            // [quads+2][8][4] column inside the box
+  uint32_t fzero = 0;                  // first of the two quads of zeros
   uint32_t* brow = nullptr;            // [nseg] device row of each piece (backward order)
-  uint32_t* pchunk = nullptr;          // [npanels+1] first chunk of each box
-  uint2* chunk = nullptr;              // [nchunks+1] {first piece, first element}
-  uint16_t* boff = nullptr;            // [nchunks*(kBoxVox+1)] voxel element offsets
-  uint16_t* bpc = nullptr;             // [nnz] piece inside the chunk
-  float* bval = nullptr;               // [nnz]
+  uint32_t* pchunk = nullptr;          // [npanels+1] first backward chunk of each box
+  uint2* chunk = nullptr;              // [chunks+1] {first piece, first element}
+  uint16_t* boff = nullptr;            // [chunks*(kBoxVox+1)] voxel element offsets
+  uint16_t* bpc = nullptr;             // piece of each element inside its chunk
+  float* bval = nullptr;               // value of each element
   uint32_t* colslot = nullptr;         // [cols+1] slot of each panel-order column (identity)
   double build_seconds = 0.0;
   PanelFormat() = default;
@@ -347,20 +353,15 @@ void launch_scale_rows(const DevMatrix& m, float* r, hipStream_t s);
 // tiling; free_panels releases it.
 const PanelFormat& ensure_panels(DevMatrix& m);
 void free_panels(DevMatrix& m);
-// part[fslot * W + f] = piece dot products with X (panel order, [cols][W]);
-// part[c * W + f] = (A^T R)_c for every panel-order column c, R [rows][W] in
-// device row order (one slot per column: colslot is the identity).
-// One workgroup per box; grid is not used. For W <= 8 (panel_slots_by_box)
-// the forward writes piece s (forward order) to part[s * W + f] instead, so
-// that a box's sums are written contiguously; the slot sums of row r then
-// read part[rowpiece[k] * W + f] for k in [rowslot[r], rowslot[r+1]).
-constexpr bool panel_slots_by_box(int W) { return W <= 8; }
+// part[s * W + f] = dot product of piece s with X (panel order, [cols][W]); a
+// row's pieces are rowpiece[rowslot[r]] .. rowpiece[rowslot[r + 1] - 1].
+// Slots are numbered box by box in chunks of rows, so that neighbouring rows'
+// slots lie together. U[c * W + f] = (A^T R)_c for every panel-order column c,
+// R [rows][W] in device row order. One workgroup per box.
 template <int W>
-void launch_panel_fwd(const PanelFormat& P, const float* X, float* part, uint32_t grid,
-                      hipStream_t s);
+void launch_panel_fwd(const PanelFormat& P, const float* X, float* part, hipStream_t s);
 template <int W>
-void launch_panel_bwd(const PanelFormat& P, const float* R, float* part, uint32_t grid,
-                      hipStream_t s);
+void launch_panel_bwd(const PanelFormat& P, const float* R, float* U, hipStream_t s);
 // ---- load-time layout (layout.hip) ----------------------------------------
 // Renumber rows (sinogram order) and voxels (4x4x2 bricks) when the grid is
 // known, build the CSC (file row order inside every column) and the

@@ -237,15 +237,13 @@ void build_host_panels(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_
   rseg[nseg] = (uint32_t)nnz;
 
   const int TP = std::max(1, std::min<int>(T, (int)std::max<uint32_t>(P, 1)));
-  // ---- forward: inside every box the pieces longest first (stable)
   // Chunks of both directions start at multiples of kFAlign / kBAlign
-  // elements, so that their elements load in 16-byte pieces; the gaps hold
-  // zero values (column / piece 0), and the arrays end with a chunk's worth
-  // of zeros so that whole-chunk loads stay inside them.
+  // elements; the gaps hold zero values (column / piece 0), and the arrays end
+  // with a chunk's worth of zeros.
   auto align_up = [](uint64_t x, uint64_t a) { return (x + a - 1) / a * a; };
-  // ---- forward: inside every box the pieces longest first (stable), cut
-  // greedily into chunks of at most kFChunkPieces pieces / kFChunkElems
-  // elements
+  // ---- forward: every box's pieces (rows ascending) cut greedily into chunks
+  // of at most kFChunkPieces pieces / kFChunkElems elements, the pieces of a
+  // chunk longest first (stable)
   std::vector<std::vector<uint32_t>> forder(P), fcut(P);
   std::vector<uint64_t> fsize(P, 0);
   parallel_for(TP, [&](int t) {
@@ -254,16 +252,16 @@ void build_host_panels(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_
       std::vector<uint32_t>& idx = forder[p];
       idx.resize(s1 - s0);
       std::iota(idx.begin(), idx.end(), s0);
-      std::stable_sort(idx.begin(), idx.end(), [&](uint32_t a, uint32_t b) {
-        return rseg[a + 1] - rseg[a] > rseg[b + 1] - rseg[b];
-      });
       uint64_t size = 0;
       for (uint32_t i = 0; i < s1 - s0;) {
         fcut[p].push_back(i);
         uint32_t n = 0, j = i;
         while (j < s1 - s0 && j - i < kFChunkPieces &&
-               n + (rseg[idx[j] + 1] - rseg[idx[j]]) <= kFChunkElems)
-          n += rseg[idx[j] + 1] - rseg[idx[j]], ++j;
+               n + (rseg[s0 + j + 1] - rseg[s0 + j]) <= kFChunkElems)
+          n += rseg[s0 + j + 1] - rseg[s0 + j], ++j;
+        std::stable_sort(idx.begin() + i, idx.begin() + j, [&](uint32_t a, uint32_t b) {
+          return rseg[a + 1] - rseg[a] > rseg[b + 1] - rseg[b];
+        });
         size += align_up(n, kFAlign);
         i = j;
       }

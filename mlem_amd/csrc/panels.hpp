@@ -15,17 +15,17 @@
 //   the box.
 //
 //   forward (f = A X): a workgroup loads its box's slice of X into LDS and
-//   writes one W-wide dot product per piece into the piece's slot. The slots
-//   of one row are contiguous, in box order, so a second pass adds them in a
-//   fixed order. Inside a box the pieces are stored longest first, so the
-//   lanes of a wave get pieces of about the same length, and staged in LDS
-//   in chunks (at most 256 pieces and 4096 elements).
+//   writes one W-wide dot product per piece into the piece's slot; a second
+//   pass adds a row's slots in box order. The box's pieces, rows ascending, are
+//   cut into chunks of at most 1024 pieces; inside a chunk they are stored
+//   longest first, so the lanes of a wave get pieces of about the same length,
+//   while the slots of neighbouring rows stay close together.
 //
 //   backward (u = A^T R): a workgroup holds its box's voxel sums in
-//   registers and walks the box's pieces (rows ascending) in chunks: the
-//   chunk's runs of R are staged in LDS, then every voxel adds its elements
-//   of the chunk (chunk order, then rows ascending). Every voxel's sum is
-//   complete at the end, one slot per voxel.
+//   registers and walks the box's pieces (rows ascending) in chunks of at most
+//   512 pieces and 8192 elements: the chunk's runs of R are staged in LDS, then
+//   every voxel adds its elements of the chunk (chunk order, then rows
+//   ascending). Every voxel's sum is complete at the end, one slot per voxel.
 //
 // Sums are deterministic (fixed order), not the sequential order of the
 // reference driver (mlem_seq/seqcsr4mlem.cpp:69-120).
@@ -40,8 +40,8 @@ constexpr uint32_t kBoxVox = 1024;      // voxels per box (at most)
 constexpr uint32_t kMaxSegment = 512;   // longer pieces are split, each with its own slot
 constexpr uint32_t kChunkPieces = 512;   // backward: pieces staged per chunk (at most)
 constexpr uint32_t kChunkElems = 8192;   // backward: elements staged per chunk (at most)
-constexpr uint32_t kFChunkPieces = 256;  // forward: pieces staged per chunk (at most)
-constexpr uint32_t kFChunkElems = 4096;  // forward: elements staged per chunk (at most)
+constexpr uint32_t kFChunkPieces = 1024; // forward: pieces per chunk (at most)
+constexpr uint32_t kFChunkElems = 16384; // forward: elements per chunk (at most)
 constexpr uint32_t kFAlign = 4;          // forward chunks start at multiples of 4 elements
 constexpr uint32_t kBAlign = 8;          // backward chunks start at multiples of 8 elements
 
@@ -52,7 +52,7 @@ struct HostPanels {
   // column order of the tiling ("panel order"): boxes one after the other
   std::vector<uint32_t> pc_of_dev;    // [cols] panel-order column of each device column
   std::vector<uint32_t> pstart;       // [npanels+1] first panel-order column of each box
-  // forward: pieces box-major, longest first inside a box
+  // forward: pieces box-major, in chunks, longest first inside a chunk
   std::vector<uint32_t> pseg;         // [npanels+1] first piece of each box
   std::vector<uint32_t> fseg;         // [nseg+1] first element of each piece
   std::vector<uint32_t> fslot;        // [nseg] row-major slot of each piece

@@ -265,12 +265,12 @@ void spmm_launch(mlem_tape* T, bool csc, const float* v, const Epi& epi) {
     const uint32_t n = csc ? m.cols : m.rows;
     float* part = csc ? T->upart : T->fpart;
     if (csc)
-      launch_panel_bwd<W>(P, v, part, T->grid, m.stream);
+      launch_panel_bwd<W>(P, v, part, m.stream);
     else
-      launch_panel_fwd<W>(P, v, part, T->grid, m.stream);
+      launch_panel_fwd<W>(P, v, part, m.stream);
     hipLaunchKernelGGL((k_slot_sums<W, Epi>), dim3(blocks_for((uint64_t)n * W)), dim3(kBlock), 0,
                        m.stream, csc ? P.colslot : P.rowslot,
-                       (!csc && panel_slots_by_box(W)) ? P.rowpiece : nullptr, n, part, epi);
+                       csc ? nullptr : P.rowpiece, n, part, epi);
   } else if (csc) {
     hipLaunchKernelGGL((k_spmm<W, Epi>), dim3(T->grid), dim3(kBlock), 0, m.stream, m.colptr, m.csc,
                        T->tiles_b, T->nt_b, v, epi);
@@ -397,7 +397,7 @@ int mlem_forward_k_mode(mlem_matrix* h, uint32_t frames, const float* y, uint32_
       T->colmap = T->P->pc_of_file;
       T->norm = T->P->norm;
       MLEM_HIP(hipMalloc(&T->fpart, 4ull * std::max<uint64_t>(T->P->nseg, 1) * W));
-      MLEM_HIP(hipMalloc(&T->upart, 4ull * std::max<uint64_t>(T->P->ngroups, 1) * W));
+      MLEM_HIP(hipMalloc(&T->upart, 4ull * std::max<uint64_t>(m.cols, 1) * W));
     }
     prepare_tiles(m, m.stream);
     if (mode == MLEM_MODE_EXACT) {  // record tiles of the sequential SpMM walker
