@@ -74,3 +74,53 @@ def test_block_images_against_fp64(grid, rows, dense, with_grid, width):
                 assert np.array_equal(got[f] == 0, ref == 0), f
                 on = ref != 0
                 assert np.abs(got[f][on] / ref[on] - 1).max() <= tol, f
+
+
+@pytest.mark.parametrize("frames", [1, 5, 13, 20])          # blocks of 4, 8, 16 and 32 frames
+@pytest.mark.parametrize("grid,rows,dense,with_grid", [
+    ((16, 16, 4), 7, False, True),          # rows of one piece
+    ((33, 31, 9), 600, True, True),         # rows of 0 to 18 pieces
+    ((33, 31, 9), 599, False, False),
+])
+def test_one_unrolled_iteration_against_fp64(grid, rows, dense, with_grid, frames):
+    rowidx, el, cols = _matrix(grid, rows, dense, rows + frames)
+    rng = np.random.default_rng(4)
+    Y = rng.uniform(0.5, 20.0, (frames, rows)).astype(np.float32)
+    X0 = rng.uniform(0.5, 2.0, (frames, cols)).astype(np.float32)
+    G = rng.uniform(0.5, 2.0, (frames, cols)).astype(np.float32)
+    lengths = np.diff(np.concatenate([[0], rowidx.astype(np.int64)]))
+    hits = np.bincount(el["column"], minlength=cols)
+    rowof = np.repeat(np.arange(rows), lengths)
+    a = el["value"].astype(np.float64)
+
+    def fwd(v):
+        return np.bincount(rowof, a * v[el["column"]], rows)
+
+    def bwd(r):
+        return np.bincount(el["column"], a * r[rowof], cols)
+
+    # Positive terms throughout (n-1 roundings for a sum of n terms, 2^-24
+    # each): f and A(g x/n) have at most `longest` terms, n, u and A'(gf) at
+    # most `most`; every output passes through at most three of each kind and
+    # a dozen single operations. The gradient of the image is a difference of
+    # two such terms: the bound is relative to their sum.
+    tol = (3 * (lengths.max() + hits.max()) + 12) * 2.0 ** -24
+    with M.Csr4Matrix.from_arrays(rows, cols, rowidx, el, grid=grid if with_grid else None) as A:
+        u = M.Unrolled(A, Y, X0, K=1, mode="fast")
+        gy, gx0 = u.backward(G)
+        for k in range(frames):
+            x, g = X0[k].astype(np.float64), G[k].astype(np.float64)
+            n = np.where(hits > 0, bwd(np.ones(rows)), 1.0)
+            f = fwd(x)
+            on = f != 0
+            fs = np.where(on, f, 1.0)
+            r = np.where(on, Y[k] / fs, 0.0)
+            b = bwd(r)
+            gr = fwd(g * x / n)
+            xK = orc.f64_unroll(rowidx, el, cols, Y[k], X0[k], 1)
+            assert np.all(np.abs(u.xK[k] - xK) <= tol * np.abs(xK))
+            want = np.where(on, gr / fs, 0.0)
+            assert np.all(np.abs(gy[k] - want) <= tol * want)
+            back = bwd(np.where(on, gr * r / fs, 0.0))
+            assert np.all(np.abs(gx0[k] - (g * b / n - back)) <= tol * (g * b / n + back))
+        u.close()
