@@ -345,13 +345,19 @@ std::vector<uint32_t> brick_colmap(uint32_t nx, uint32_t ny, uint32_t nz) {
 }
 
 namespace {
+// The sorts by column merge up to 131072 records and go digit by digit above
+// (the library's own line is 1048576): a 2 MB block of 219000 records 124
+// instead of 152 us a block and iteration, 8 MB 168 instead of 252, while a block
+// of 77000 takes 130 digit by digit and 112 merged.
+using ColumnSort = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
+                                              rocprim::default_config, 131072>;
 size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
 size_t block_csc_sort_bytes(uint64_t nnz, uint32_t cols) {
   size_t tb = 0;
-  MLEM_HIP(rocprim::radix_sort_pairs(nullptr, tb, (uint32_t*)nullptr, (uint32_t*)nullptr,
-                                     (unsigned long long*)nullptr, (unsigned long long*)nullptr,
-                                     (size_t)nnz, 0, bits_for(cols ? cols - 1 : 0),
-                                     hipStream_t(nullptr)));
+  MLEM_HIP(rocprim::radix_sort_pairs<ColumnSort>(
+      nullptr, tb, (uint32_t*)nullptr, (uint32_t*)nullptr, (unsigned long long*)nullptr,
+      (unsigned long long*)nullptr, (size_t)nnz, 0, bits_for(cols ? cols - 1 : 0),
+      hipStream_t(nullptr)));
   return tb;
 }
 }  // namespace
@@ -380,9 +386,9 @@ void build_block_csc(const uint32_t* rowptr, const uint2* csr, uint32_t rows, ui
   hipLaunchKernelGGL(k_csc_keys, dim3(blocks_for((uint64_t)rows * 16)), dim3(kBlock), 0, s, rowptr,
                      csr, rows, (const uint32_t*)nullptr, (const uint32_t*)nullptr, keys, vals);
   check_launch("block csc key launch");
-  MLEM_HIP(rocprim::radix_sort_pairs(temp, tb, keys, skeys, vals,
-                                     reinterpret_cast<unsigned long long*>(csc), (size_t)nnz, 0,
-                                     bits_for(cols ? cols - 1 : 0), s));
+  MLEM_HIP(rocprim::radix_sort_pairs<ColumnSort>(
+      temp, tb, keys, skeys, vals, reinterpret_cast<unsigned long long*>(csc), (size_t)nnz, 0,
+      bits_for(cols ? cols - 1 : 0), s));
   hipLaunchKernelGGL(k_colptr_search, dim3(blocks_for((uint64_t)cols + 1)), dim3(kBlock), 0, s,
                      skeys, nnz, cols, colptr);
   check_launch("block colptr launch");
@@ -447,12 +453,12 @@ void build_layout(DevMatrix& m, bool reorder_rows, bool reorder_cols, bool want_
       const int end_bit = bits_for(m.cols - 1);
       size_t tb = 0;
       auto* out = reinterpret_cast<unsigned long long*>(m.csc);
-      MLEM_HIP(rocprim::radix_sort_pairs(nullptr, tb, keys.as<uint32_t>(), skeys.as<uint32_t>(),
-                                         vals.as<unsigned long long>(), out, (size_t)m.nnz, 0,
+      MLEM_HIP(rocprim::radix_sort_pairs<ColumnSort>(nullptr, tb, keys.as<uint32_t>(),
+                                         skeys.as<uint32_t>(), vals.as<unsigned long long>(), out, (size_t)m.nnz, 0,
                                          end_bit, s));
       temp.alloc(tb);
-      MLEM_HIP(rocprim::radix_sort_pairs(temp.p, tb, keys.as<uint32_t>(), skeys.as<uint32_t>(),
-                                         vals.as<unsigned long long>(), out, (size_t)m.nnz, 0,
+      MLEM_HIP(rocprim::radix_sort_pairs<ColumnSort>(temp.p, tb, keys.as<uint32_t>(),
+                                         skeys.as<uint32_t>(), vals.as<unsigned long long>(), out, (size_t)m.nnz, 0,
                                          end_bit, s));
       hipLaunchKernelGGL(k_colptr, dim3(blocks_for(m.nnz)), dim3(kBlock), 0, s,
                          skeys.as<uint32_t>(), m.nnz, m.cols, m.colptr);
