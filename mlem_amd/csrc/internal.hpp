@@ -120,10 +120,39 @@ struct GroupLaunch {
 // pointers, global columns) and their transpose as CSC (global rows); a
 // projection copies its part of every block in turn through two device
 // buffers, the copy of the next block overlapping the kernels of this one.
+//
+// The CSR part of a block of at least kPackMin elements that is not resident is
+// held packed (when the device has room to unpack one), chunk by chunk of
+// kPackChunk elements:
+//   row pointers | PackHead per chunk | kPackTable column steps | chunks
+// A chunk is the elements' values, one code per element and the steps of the
+// elements with code kPackEscape, each padded to 16 bytes: the column of an
+// element is the column before it in the chunk (0 before the first) plus, modulo
+// 2^32, the step of its code. A chunk that would not become smaller holds the
+// 8-byte records (steps = kPackRaw).
+//
+// Why from 2^20 elements on: below, a block's kernels take longer than the copy of
+// its 8-byte records (8 MB: 168 us against 160; 4 MB: 145 against 80), and
+// unpacking would only add to them (77000 elements: 100 to 112 us a block).
+// Above, the copy is what counts: 96x96x40 voxels, 700001 lines, 5 iterations take
+// 51.5 ms from 64 MB blocks of records and 34.8 packed (5.1 bytes per element),
+// 60.5 and 48.6 from 12 MB blocks.
+constexpr uint64_t kPackMin = 1u << 20;
+constexpr uint32_t kPackChunk = 4096;
+constexpr uint32_t kPackTable = 256;
+constexpr uint32_t kPackEscape = 255;
+constexpr uint32_t kPackRaw = 0xFFFFFFFFu;
+struct PackHead {
+  uint32_t at;     // 16-byte units from the first chunk
+  uint32_t count;  // elements
+  uint32_t steps;  // escaped steps, or kPackRaw
+  uint32_t pad;
+};
 struct StreamBlock {
   uint32_t row0 = 0, rows = 0;  // first row, rows
   uint64_t nnz = 0;
   uint64_t csr_off = 0, csr_bytes = 0;  // parts within the host buffer
+  uint64_t packed_bytes = 0;            // of the packed CSR part; 0: not packed
   uint64_t csc_off = 0, csc_bytes = 0;
   char* resident = nullptr;  // device copy of both parts (CSR, then CSC), or none
 };
@@ -145,6 +174,7 @@ struct StreamedMatrix {
   char* csc_dev = nullptr;
   uint64_t csc_scratch_bytes = 0;
   uint64_t max_stream_nnz = 0;
+  uint2* expand = nullptr;  // [max_stream_nnz] elements of the block unpacked last
   StreamedMatrix() = default;
   StreamedMatrix(const StreamedMatrix&) = delete;
   StreamedMatrix& operator=(const StreamedMatrix&) = delete;
@@ -331,6 +361,8 @@ size_t block_csc_scratch(uint64_t nnz, uint32_t cols);
 void build_block_csc(const uint32_t* rowptr, const uint2* csr, uint32_t rows, uint32_t cols,
                      uint64_t nnz, void* scratch, size_t scratch_bytes, uint32_t* colptr,
                      uint2* csc, hipStream_t s);
+// Elements of a packed block: heads, steps table and chunks as they arrived.
+void launch_unpack(const PackHead* heads, uint64_t nnz, uint2* el, hipStream_t s);
 // x *= (n != 0) ? u/n : u; optionally u = 0 afterwards.
 void launch_update(uint32_t cols, const float* u, const float* norm, float* x,
                    bool zero_u, hipStream_t s);

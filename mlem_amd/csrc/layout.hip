@@ -345,6 +345,87 @@ std::vector<uint32_t> brick_colmap(uint32_t nx, uint32_t ny, uint32_t nz) {
 }
 
 namespace {
+// One packed chunk (PackHead) per workgroup, 16 elements per lane: the codes'
+// steps, escapes taken in order, then the running sum over the chunk.
+//
+// Bound by its 13 bytes per element (5 read, 8 written): 34 us for 8.2M elements,
+// 3.1 TB/s. The chunk's columns go through LDS so that the records are written
+// in runs.
+__global__ __launch_bounds__(kBlock) void k_unpack(const PackHead* __restrict__ heads,
+                                                   const uint32_t* __restrict__ table,
+                                                   const char* __restrict__ chunks,
+                                                   uint2* __restrict__ el) {
+  constexpr uint32_t E = kPackChunk / kBlock;  // elements per lane
+  static_assert(E == 16 && kPackTable == kBlock, "a lane loads 16 codes and one step");
+  // fewer escapes than this, or the chunk is not smaller than its records
+  constexpr uint32_t kMaxSteps = 3 * kPackChunk / 4;
+  __shared__ uint32_t step[kPackTable];
+  __shared__ uint32_t esc[kMaxSteps];
+  __shared__ uint32_t col[kPackChunk + kPackChunk / E];
+  __shared__ uint32_t wsum[2][kBlock / 64];
+  const uint32_t t = threadIdx.x, lane = t % 64, wave = t / 64;
+  const PackHead h = heads[blockIdx.x];
+  const uint32_t m = h.count;
+  const char* __restrict__ p = chunks + 16ull * h.at;
+  uint2* __restrict__ out = el + (size_t)blockIdx.x * kPackChunk;
+  if (h.steps == kPackRaw) {
+    for (uint32_t i = t; i < m; i += kBlock) out[i] = reinterpret_cast<const uint2*>(p)[i];
+    return;
+  }
+  const uint32_t vb = (4 * m + 15) & ~15u, cb = (m + 15) & ~15u;
+  const float* __restrict__ val = reinterpret_cast<const float*>(p);
+  step[t] = table[t];
+  for (uint32_t i = t; i < h.steps; i += kBlock)
+    esc[i] = reinterpret_cast<const uint32_t*>(p + vb + cb)[i];
+  uint4 c4 = make_uint4(0, 0, 0, 0);  // (padding codes are 0)
+  if (E * t < cb) c4 = reinterpret_cast<const uint4*>(p + vb)[t];
+  const uint32_t c[4] = {c4.x, c4.y, c4.z, c4.w};
+  uint32_t ne = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < E; ++k) ne += ((c[k / 4] >> (8 * (k % 4))) & 0xFFu) == kPackEscape;
+  // sum over the lanes before this one
+  auto before = [&](uint32_t x, uint32_t* ws) __attribute__((always_inline)) {
+    uint32_t run = x;
+#pragma unroll
+    for (uint32_t d = 1; d < 64; d <<= 1) {
+      const uint32_t o = (uint32_t)__shfl_up((int)run, d);
+      if (lane >= d) run += o;
+    }
+    if (lane == 63) ws[wave] = run;
+    __syncthreads();
+    uint32_t base = run - x;
+    for (uint32_t w = 0; w < wave; ++w) base += ws[w];
+    return base;
+  };
+  uint32_t at = before(ne, wsum[0]);  // (its barrier also covers step and esc)
+  uint32_t s[E], sum = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < E; ++k) {
+    const uint32_t code = (c[k / 4] >> (8 * (k % 4))) & 0xFFu;
+    if (code == kPackEscape)
+      sum += esc[at++];
+    else
+      sum += step[code];
+    s[k] = sum;
+  }
+  const uint32_t base = before(sum, wsum[1]);
+#pragma unroll
+  for (uint32_t k = 0; k < E; ++k) col[t * (E + 1) + k] = base + s[k];
+  __syncthreads();
+  for (uint32_t i = t; i < m; i += kBlock)
+    out[i] = make_uint2(col[i + i / E], __float_as_uint(val[i]));
+}
+}  // namespace
+
+void launch_unpack(const PackHead* heads, uint64_t nnz, uint2* el, hipStream_t s) {
+  const uint32_t n = (uint32_t)((nnz + kPackChunk - 1) / kPackChunk);
+  const uint32_t* table = reinterpret_cast<const uint32_t*>(heads + n);
+  hipLaunchKernelGGL(k_unpack, dim3(n), dim3(kBlock), 0, s, heads, table,
+                     reinterpret_cast<const char*>(table + kPackTable), el);
+  check_launch("unpack launch");
+}
+
+namespace {
 // The sorts by column merge up to 131072 records and go digit by digit above
 // (the library's own line is 1048576): a 2 MB block of 219000 records 124
 // instead of 152 us a block and iteration, 8 MB 168 instead of 252, while a block

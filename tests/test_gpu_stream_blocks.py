@@ -1,5 +1,8 @@
-"""Streamed matrices in small blocks: EXACT iterations against the fp32
-restatement, bit for bit."""
+"""Streamed blocks packed to column codes: EXACT projections and iterations
+(every element's row, column and value used once, in order) against the fp32
+restatement, bit for bit: blocks on both sides of the smallest packed size,
+whole and partial last chunks of 4096 elements, columns that pack and columns
+that do not, blocks resident or not."""
 from __future__ import annotations
 
 import numpy as np
@@ -11,6 +14,7 @@ from oracle import oracle as orc
 pytestmark = pytest.mark.gpu
 
 CHUNK = 4096
+MIN = 1 << 20          # elements of the smallest block that is packed
 
 
 def _matrix(kind, nnz, cols, seed):
@@ -32,6 +36,28 @@ def _matrix(kind, nnz, cols, seed):
     el["column"] = c
     el["value"] = rng.random(nnz, dtype=np.float32) + np.float32(0.1)
     return rows, rowidx, el
+
+
+@pytest.mark.parametrize("resident", [False, True])
+@pytest.mark.parametrize("kind,cols", [("steps", 1), ("steps", 7001), ("many", 90001),
+                                       ("random", 90001), ("mixed", 30011)])
+@pytest.mark.parametrize("nnz", [MIN - 1, MIN, MIN + 1, MIN + CHUNK - 1, 3 * MIN + 777])
+def test_exact_results_of_packed_blocks(nnz, kind, cols, resident):
+    rows, rowidx, el = _matrix(kind, nnz, cols, nnz + cols)
+    rng = np.random.default_rng(5)
+    x = rng.random(cols, dtype=np.float32) + np.float32(0.5)
+    r = rng.random(rows, dtype=np.float32)
+    y = rng.poisson(30.0, rows).astype(np.int32)
+    # one block, or two packed ones and a smaller last one that is not
+    block = 4 * (max(rows, cols) + 64) + 8 * (MIN + MIN // 3)
+    keep = 2 * block if resident else 0              # the first block stays on the device
+    with M.Csr4Matrix.from_arrays(rows, cols, rowidx, el, stream_block_bytes=block,
+                                  stream_resident_bytes=keep) as A:
+        assert A.stream_blocks() == (3 if nnz > 2 * MIN else 1)
+        assert np.array_equal(M.calcFwProj(A, x, mode="exact"), orc.fwproj(rowidx, el, x))
+        assert np.array_equal(M.calcBkProj(A, r, mode="exact"), orc.bkproj(rowidx, el, r, cols))
+        assert np.array_equal(M.mlem(A, y, None, 3, mode="exact"),
+                              orc.mlem(rowidx, el, cols, y, 3)[0])
 
 
 # The transpose of small blocks is sorted by merging up to 131072 elements and
