@@ -444,8 +444,7 @@ void enqueue_iteration(mlem_recon* R) {
   } else if (m.streamed) {
     stream_iteration(m, R->mode, R->x, R->y, R->r, st, m.stream);
   } else {
-    launch_fwd(m, R->mode, R->x, R->y, R->r, true, st, m.stream);
-    launch_bwd(m, R->mode, R->r, m.norm, R->x, true, m.stream);
+    launch_iteration(m, R->mode, R->x, R->y, R->r, st, m.stream);
   }
 }
 

@@ -605,8 +605,7 @@ void launch_single(mlem_batch* B, RhsBlock& b, hipStream_t s) {
   st.results = b.results;
   st.ring = kRing;
   st.max_blocks = b.pmax;
-  launch_fwd(m, B->mode, b.X, b.Y, b.R, true, &st, s);
-  launch_bwd(m, B->mode, b.R, m.norm, b.X, true, s);
+  launch_iteration(m, B->mode, b.X, b.Y, b.R, &st, s);
 }
 
 void launch_any(mlem_batch* B, RhsBlock& b, hipStream_t s, int set) {

@@ -319,6 +319,10 @@ void launch_fwd(const DevMatrix& m, int mode, const float* x, const int32_t* y,
 // `out` (which holds x), else out = u.
 void launch_bwd(const DevMatrix& m, int mode, const float* r, const float* norm,
                 float* out, bool update, hipStream_t s);
+// One iteration: r = y / (A x), x *= (A^T r) / norm. The statistics of the
+// forward projection (or nullptr) are complete after both.
+void launch_iteration(const DevMatrix& m, int mode, float* x, const int32_t* y, float* r,
+                      const StatsState* stats, hipStream_t s);
 // Backprojection by atomic scatter over the CSR: u += A^T r (u pre-zeroed).
 void launch_scatter(const DevMatrix& m, const float* r, float* u, hipStream_t s);
 // One row block of a streamed matrix (kernels.hip).

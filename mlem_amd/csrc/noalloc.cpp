@@ -104,8 +104,7 @@ int mlem_reconstruct_noalloc(mlem_matrix* h, const int32_t* y, uint32_t rows, fl
     launch_fill(reinterpret_cast<float*>(st.counter), 0.f, 2, s);
     double2 res[kRing];
     for (int k = 0; k < iterations; ++k) {
-      launch_fwd(m, mode, xs, ys, rs, true, stats ? &st : nullptr, s);
-      launch_bwd(m, mode, rs, m.norm, xs, true, s);
+      launch_iteration(m, mode, xs, ys, rs, stats ? &st : nullptr, s);
       if (stats && ((k + 1) % (int)kRing == 0 || k + 1 == iterations)) {
         const int first = k - k % (int)kRing, n = k + 1 - first;
         MLEM_HIP(hipMemcpyAsync(res, st.results, sizeof(double2) * n, hipMemcpyDeviceToHost, s));
