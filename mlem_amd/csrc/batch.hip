@@ -12,9 +12,8 @@
 // by the epilogue kernel k_tiled_ratio (ratio and statistics), and complete
 // per-voxel backprojections, applied by k_tiled_update (masked update);
 // deterministic, not the reference's summation order.
-// MLEM_MODE_EXACT: each 256-lane block walks whole tiles of rows (CSC
-// columns), stages the tile's 8-byte records in LDS with coalesced loads, and
-// gives every row (column) to a group of W lanes, lane f accumulating frame f
+// MLEM_MODE_EXACT: every row (CSC column) belongs to a group of W lanes
+// (spmm.hpp), lane f accumulating frame f
 // sequentially in file element order with separate multiply and add: per
 // frame, the result is bit-identical to the reference's sequential driver
 // (mlem_seq/seqcsr4mlem.cpp:69-134).
@@ -149,14 +148,14 @@ struct BwdUpdate {
 };
 
 // Forward projection + ratio for one RHS block (f kept in Fp).
-template <int W>
+template <int W, bool kDirect>
 __global__ __launch_bounds__(kBlock) void k_fwd_batch(
     const uint32_t* __restrict__ rowptr, const uint2* __restrict__ csr,
-    const uint2* __restrict__ tiles, uint32_t ntiles,
+    const uint2* __restrict__ tiles, uint32_t count,
     const float* __restrict__ X, const int32_t* __restrict__ Y, float* __restrict__ R,
     float* __restrict__ Fp) {
   FwdRatio<W> epi{Y, R, Fp};
-  spmm::walk<W>(rowptr, csr, tiles, ntiles, X, epi);
+  spmm::product<W, kDirect>(rowptr, csr, tiles, count, X, epi);
 }
 
 // Per-frame FP64 statistics of a block's forward projection: lane f of row
@@ -181,15 +180,15 @@ __global__ __launch_bounds__(kBlock) void k_batch_loglik(const float* __restrict
   batch_stats_partial<W>(ll, tot, partials);
 }
 
-// Backprojection + update for one RHS block over the CSC column tiles.
-template <int W>
+// Backprojection + update for one RHS block over the CSC columns.
+template <int W, bool kDirect>
 __global__ __launch_bounds__(kBlock) void k_bwd_batch(
     const uint32_t* __restrict__ colptr, const uint2* __restrict__ csc,
-    const uint2* __restrict__ tiles, uint32_t ntiles,
+    const uint2* __restrict__ tiles, uint32_t count,
     const float* __restrict__ R, const float* __restrict__ norm, float* __restrict__ X,
     const uint32_t* __restrict__ mask) {
   BwdUpdate<W> epi{norm, X, *mask};
-  spmm::walk<W>(colptr, csc, tiles, ntiles, R, epi);
+  spmm::product<W, kDirect>(colptr, csc, tiles, count, R, epi);
 }
 
 // The tiled (FAST) epilogues give each lane four right-hand sides (16-byte
@@ -583,14 +582,26 @@ void launch_block(mlem_batch* B, RhsBlock& b, hipStream_t s, int set = 0) {
     return;
   }
   const DevMatrix& m = B->mat->m;
-  hipLaunchKernelGGL((k_fwd_batch<W>), dim3(B->grid), dim3(kBlock), 0, s, m.rowptr, m.csr,
-                     B->tiles_f, B->nt_f, b.X, b.Y, b.R, b.F);
+  auto fwd = [&](auto direct, uint32_t grid) {
+    hipLaunchKernelGGL((k_fwd_batch<W, direct.value>), dim3(grid), dim3(kBlock), 0, s, m.rowptr,
+                       m.csr, B->tiles_f, direct.value ? m.rows : B->nt_f, b.X, b.Y, b.R, b.F);
+  };
+  auto bwd = [&](auto direct, uint32_t grid) {
+    hipLaunchKernelGGL((k_bwd_batch<W, direct.value>), dim3(grid), dim3(kBlock), 0, s, m.colptr,
+                       m.csc, B->tiles_b, direct.value ? m.cols : B->nt_b, b.R, m.norm, b.X, b.mask);
+  };
+  if (spmm::direct<W>(false, m.cols))
+    fwd(std::bool_constant<spmm::kDirectWidth<W>>(), spmm::direct_grid<W>(m.rows));
+  else
+    fwd(std::false_type(), B->grid);
   hipLaunchKernelGGL((k_batch_loglik<W>), dim3(B->grid), dim3(kBlock), 0, s, b.F, b.Y, m.rows,
                      b.partials);
   hipLaunchKernelGGL((k_batch_stats_reduce<W>), dim3(1), dim3(kReduceLanes), 0, s, b.partials,
                      B->grid, b.counter, b.results, kRing);
-  hipLaunchKernelGGL((k_bwd_batch<W>), dim3(B->grid), dim3(kBlock), 0, s, m.colptr, m.csc,
-                     B->tiles_b, B->nt_b, b.R, m.norm, b.X, b.mask);
+  if (spmm::direct<W>(true, m.rows))
+    bwd(std::bool_constant<spmm::kDirectWidth<W>>(), spmm::direct_grid<W>(m.cols));
+  else
+    bwd(std::false_type(), B->grid);
 }
 
 // A block of one frame: the single-image EXACT projections (forward with the

@@ -11,12 +11,14 @@
 // order with separate multiply and add (this code is compiled with
 // -ffp-contract=off), so every vector's result is the reference driver's
 // sequential fp32 sum (mlem_seq/seqcsr4mlem.cpp:69-91 for the CSR,
-// :108-120 for the CSC in ascending row order).
+// :108-120 for the CSC in ascending row order). Where that is faster, the lanes
+// of a segment read its records themselves (walk_direct): the same sums.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 #include <vector>
 
 namespace mlem {
@@ -87,6 +89,88 @@ __device__ __forceinline__ void walk(const uint32_t* __restrict__ ptr,
       epi(s0 + sg, f, d);
     }
   }
+}
+
+// The same sums without tiles, for W = 16 and 32: the W lanes of a segment load
+// 16 records at a time themselves (one per lane; W = 32: both rows of 16 lanes the
+// same ones) and broadcast them along the row, the next 16 in flight while these
+// are gathered. Workgroup b takes kBlock / W neighbouring segments, numbered as
+// walk() numbers its tiles. The gathered vectors are shorter than 2^32 bytes.
+//
+// Bound by the gathered lines (64 or 128 bytes per record). No barrier and no
+// second reading of the records from LDS; but a run of 16 records is only half
+// or a whole line, read by as many waves as there are segments in it. us, walk()
+// first: A v, 128x128x48 voxels and 1327104 lines, W = 16 1622 > 1294, W = 32
+// 2395 > 1589; 75x77x31 and 200003 138 > 135, 217 > 178. A^T v, W = 32 1964 >
+// 1840, 192 > 167; but W = 16 1447 > 1635, 124 > 136, and narrower blocks 3 to
+// 20 % slower in either direction: direct() leaves those to walk().
+template <int j>
+__device__ __forceinline__ uint32_t row_lane(uint32_t x) {  // lane j of each row of 16
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x150 + j, 0xF, 0xF, true);
+}
+template <int j>
+__device__ __forceinline__ void row_gather(uint32_t at, uint32_t val, const char* __restrict__ v,
+                                           uint32_t f4, float (&g)[16], float (&a)[16]) {
+  if constexpr (j < 16) {
+    g[j] = *reinterpret_cast<const float*>(v + (row_lane<j>(at) + f4));
+    a[j] = __uint_as_float(row_lane<j>(val));
+    row_gather<j + 1>(at, val, v, f4, g, a);
+  }
+}
+template <int W, class Epi>
+__device__ __forceinline__ void walk_direct(const uint32_t* __restrict__ ptr,
+                                            const uint2* __restrict__ el, uint32_t n,
+                                            const float* __restrict__ v, Epi& epi) {
+  static_assert(W == 16 || W == 32, "whole rows of 16 lanes per segment");
+  constexpr uint32_t G = kBlock / W;
+  const uint32_t t = threadIdx.x, f = t % W, l = t % 16;
+  const uint32_t nb = (n + G - 1) / G, xcd = blockIdx.x & 7u;
+  const uint32_t blk = (uint32_t)((uint64_t)nb * xcd / 8) + (blockIdx.x >> 3);
+  const uint64_t s = (uint64_t)blk * G + t / W;
+  if (blk >= (uint32_t)((uint64_t)nb * (xcd + 1) / 8) || s >= n) return;
+  const uint32_t b = ptr[s], e = ptr[s + 1];
+  const char* __restrict__ vb = reinterpret_cast<const char*>(v);
+  float acc = 0.f;
+  uint2 next = make_uint2(0, 0);
+  if (b < e) next = el[min(b + l, e - 1)];
+  for (uint32_t k = b; k < e; k += 16) {
+    float g[16], a[16];
+    row_gather<0>(next.x * (4 * W), next.y, vb, f * 4, g, a);
+    if (k + 16 < e) next = el[min(k + 16 + l, e - 1)];
+    if (k + 16 <= e) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc = acc + a[j] * g[j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        if (k + j < e) acc = acc + a[j] * g[j];
+    }
+  }
+  epi((uint32_t)s, f, acc);
+}
+
+// count: segments (kDirect) or tiles.
+template <int W, bool kDirect, class Epi>
+__device__ __forceinline__ void product(const uint32_t* __restrict__ ptr,
+                                        const uint2* __restrict__ el,
+                                        const uint2* __restrict__ tiles, uint32_t count,
+                                        const float* __restrict__ v, Epi& epi) {
+  if constexpr (kDirect)
+    walk_direct<W>(ptr, el, count, v, epi);
+  else
+    walk<W>(ptr, el, tiles, count, v, epi);
+}
+// Whether A v (csc = false, gathering cols runs) or A^T v (csc, rows runs) of W
+// vectors takes walk_direct(); the reasons stand there.
+template <int W>
+constexpr bool kDirectWidth = W == 16 || W == 32;
+template <int W>
+inline bool direct(bool csc, uint64_t gathered) {
+  return (W == 32 || (W == 16 && !csc)) && gathered * W * 4 < (1ull << 32);
+}
+template <int W>
+inline uint32_t direct_grid(uint32_t n) {
+  return ((n + kBlock / W - 1) / (kBlock / W) + 7) / 8 * 8;
 }
 
 // Greedy partition of segments [0, n) into tiles of at most T records and

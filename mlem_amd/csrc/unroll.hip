@@ -153,12 +153,12 @@ struct AdjBwd {
   }
 };
 
-template <int W, class Epi>
+template <int W, bool kDirect, class Epi>
 __global__ __launch_bounds__(kBlock) void k_spmm(const uint32_t* __restrict__ ptr,
                                                  const uint2* __restrict__ el,
-                                                 const uint2* __restrict__ tiles, uint32_t ntiles,
+                                                 const uint2* __restrict__ tiles, uint32_t count,
                                                  const float* __restrict__ v, Epi epi) {
-  spmm::walk<W>(ptr, el, tiles, ntiles, v, epi);
+  spmm::product<W, kDirect>(ptr, el, tiles, count, v, epi);
 }
 
 // Fixed-order sums of a tiled product's partials: lane (r, q) adds quad q of
@@ -334,12 +334,17 @@ void spmm_launch(mlem_tape* T, bool csc, const float* v, const Epi& epi) {
     hipLaunchKernelGGL((k_slot_sums<W, Epi>), dim3(blocks_for((uint64_t)n * (W / 4))),
                        dim3(kBlock), 0, m.stream, csc ? P.colslot : P.rowslot,
                        csc ? nullptr : P.rowpiece, n, part, epi);
-  } else if (csc) {
-    hipLaunchKernelGGL((k_spmm<W, Epi>), dim3(T->grid), dim3(kBlock), 0, m.stream, m.colptr, m.csc,
-                       T->tiles_b, T->nt_b, v, epi);
   } else {
-    hipLaunchKernelGGL((k_spmm<W, Epi>), dim3(T->grid), dim3(kBlock), 0, m.stream, m.rowptr, m.csr,
-                       T->tiles_f, T->nt_f, v, epi);
+    const uint32_t* ptr = csc ? m.colptr : m.rowptr;
+    const uint2* el = csc ? m.csc : m.csr;
+    const uint2* tiles = csc ? T->tiles_b : T->tiles_f;
+    const uint32_t nt = csc ? T->nt_b : T->nt_f, n = csc ? m.cols : m.rows;
+    if (spmm::direct<W>(csc, csc ? m.rows : m.cols))
+      hipLaunchKernelGGL((k_spmm<W, spmm::kDirectWidth<W>, Epi>), dim3(spmm::direct_grid<W>(n)),
+                         dim3(kBlock), 0, m.stream, ptr, el, tiles, n, v, epi);
+    else
+      hipLaunchKernelGGL((k_spmm<W, false, Epi>), dim3(T->grid), dim3(kBlock), 0, m.stream, ptr, el,
+                         tiles, nt, v, epi);
   }
   ++T->spmm_launches;
 }
