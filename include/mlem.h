@@ -420,6 +420,10 @@ MLEM_API void mlem_tape_destroy(mlem_tape* t);
  *   MLEM_KERNEL_DICT_WIDE param = elements per lane (16, 24 or 32): the same
  *                      with 512-lane blocks, tiles of at most 512*param
  *                      elements and 512 rows (columns) (default, param 32).
+ * Opening a matrix chooses the tile size by its elements; smaller tiles chosen
+ * there are cut inside the 16384-element ones, which keeps every FAST sum the
+ * same bit for bit. mlem_set_launch with the family and param that
+ * mlem_open chose (that mlem_get_launch returned) sets those tiles again.
  * No reference counterpart (the reference hard-codes 1024-thread blocks,
  * mlem_cuda/versions/version_5.cu:121-126). */
 #define MLEM_KERNEL_GROUPS 0

@@ -189,7 +189,8 @@ class Csr4Matrix:
         return {"fwd": (fam[v[0].value], v[1].value), "bwd": (fam[v[2].value], v[3].value)}
 
     def set_launch(self, fwd, bwd) -> None:
-        """fwd, bwd: (family, param) as returned by launch()."""
+        """fwd, bwd: (family, param) as returned by launch(); the ones chosen at
+        open give the tiles chosen there, and the same FAST sums."""
         fam = {"groups": 0, "tiles": 1, "dict": 2, "dict512": 3}
         check(lib().mlem_set_launch(self.handle, fam[fwd[0]], int(fwd[1]), fam[bwd[0]],
                                     int(bwd[1])))

@@ -207,6 +207,16 @@ GroupLaunch make_launch(int kind, int param) {
   return g;
 }
 
+// The launch that a kernel family and its parameter stand for on a matrix that
+// was opened with `open` for this projection: that launch itself where they name
+// it (mlem_get_launch gives a family and a parameter alone, and its tiles may be
+// nested), so that what mlem_get_launch returned can be set again with the same
+// tiles and the same FAST sums.
+GroupLaunch named_launch(int kind, int param, const GroupLaunch& open) {
+  const GroupLaunch g = make_launch(kind, param);
+  return is_dict(kind) && open.kind == kind && open.ept == param ? open : g;
+}
+
 // Dictionary tiles of a projection whose segments end at ptr. 16384-element
 // tiles run by 512-lane blocks, two per CU (LDS- and register-bound), are the
 // fastest once every CU gets several: pet (168.4M elements) forward / backward
@@ -236,12 +246,12 @@ GroupLaunch default_launch(uint64_t nnz, const std::vector<uint32_t>& ptr) {
 }
 
 // Candidate FAST-mode configurations of one projection.
-std::vector<GroupLaunch> launch_candidates() {
+std::vector<GroupLaunch> launch_candidates(const GroupLaunch& open) {
   std::vector<GroupLaunch> c;
-  for (int e : {16, 24, 32}) c.push_back(make_launch(kDictWide, e));
-  for (int e : {8, 16, 24, 32, 48, 64}) c.push_back(make_launch(kDict, e));
-  for (int e : {4, 8, 16}) c.push_back(make_launch(kTiles, e));
-  for (int g : {8, 16, 32, 64}) c.push_back(make_launch(kGroups, g));
+  for (int e : {16, 24, 32}) c.push_back(named_launch(kDictWide, e, open));
+  for (int e : {8, 16, 24, 32, 48, 64}) c.push_back(named_launch(kDict, e, open));
+  for (int e : {4, 8, 16}) c.push_back(named_launch(kTiles, e, open));
+  for (int g : {8, 16, 32, 64}) c.push_back(named_launch(kGroups, g, open));
   return c;
 }
 
@@ -267,7 +277,7 @@ void autotune(DevMatrix& m) {
   launch_fill(reinterpret_cast<float*>(y), 0.f, m.rows, m.stream);
   float best = 1e30f;
   GroupLaunch bestF = m.fwd, bestB = m.bwd;
-  for (const GroupLaunch& g : launch_candidates()) {
+  for (const GroupLaunch& g : launch_candidates(m.fwd_open)) {
     m.fwd = g;
     prepare_tiles(m, m.stream);
     const float t = time_variant(
@@ -280,7 +290,7 @@ void autotune(DevMatrix& m) {
   m.fwd = bestF;
   if (m.csc) {
     best = 1e30f;
-    for (const GroupLaunch& g : launch_candidates()) {
+    for (const GroupLaunch& g : launch_candidates(m.bwd_open)) {
       m.bwd = g;
       prepare_tiles(m, m.stream);
       const float t = time_variant(
@@ -364,8 +374,8 @@ void finish_open(mlem_matrix* h, unsigned flags) {
 
   const double avgRow = m.rows ? (double)m.nnz / m.rows : 1.0;
   download_pointers(m, m.stream);
-  m.fwd = default_launch(m.nnz, m.h_rowptr);
-  m.bwd = default_launch(m.nnz, m.h_colptr);
+  m.fwd = m.fwd_open = default_launch(m.nnz, m.h_rowptr);
+  m.bwd = m.bwd_open = default_launch(m.nnz, m.h_colptr);
   m.scatter = make_launch(kGroups, lanes_for(avgRow));
   prepare_tiles(m, m.stream);
   if (env_int("MLEM_AUTOTUNE", 0) > 0) autotune(m);
@@ -1230,7 +1240,8 @@ int mlem_set_launch(mlem_matrix* h, int fk, int fp, int bk, int bp) {
   return guarded([&] {
     if (!h) raise(MLEM_EINVAL, "null matrix handle");
     if (h->m.streamed) raise(MLEM_EINVAL, "streamed matrices have a fixed launch configuration");
-    const GroupLaunch f = make_launch(fk, fp), b = make_launch(bk, bp);
+    const GroupLaunch f = named_launch(fk, fp, h->m.fwd_open),
+                      b = named_launch(bk, bp, h->m.bwd_open);
     ++h->m.launch_gen;
     h->m.fwd = f;
     h->m.bwd = b;

@@ -253,6 +253,7 @@ struct DevMatrix {
   float* rscale = nullptr;     // [rows] device row order, nullptr for fp32
 
   GroupLaunch fwd, bwd, scatter;
+  GroupLaunch fwd_open, bwd_open;  // as chosen when the matrix was opened
   // Bumped whenever the launch configuration (and with it the tile and
   // dictionary buffers) may change; captured iterations are re-captured.
   uint64_t launch_gen = 0;
