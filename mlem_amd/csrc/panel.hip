@@ -264,12 +264,10 @@ struct Batch {
 template <int W>
 constexpr uint32_t kDepth = W == 32 ? 8 : W == 16 ? 2 : 3;
 
-// Quads of the longest octet of a wave's round. Octets are in order of length;
-// only the zero elements (fewer than 4) at the end of a chunk can make a later
-// one longer, by one quad.
+// Quads of the longest octet of a wave's round: the first lane's (octets are in
+// order of length).
 __device__ __forceinline__ uint32_t longest(uint32_t quads) {
-  const uint32_t a = __builtin_amdgcn_readfirstlane(quads);
-  return __builtin_amdgcn_ballot_w64(quads > a) ? a + 1 : a;
+  return __builtin_amdgcn_readfirstlane(quads);
 }
 
 // A piece's sums: whole 128-byte lines go past the caches (read once, by the

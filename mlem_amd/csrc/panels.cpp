@@ -237,9 +237,10 @@ void build_host_panels(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_
   rseg[nseg] = (uint32_t)nnz;
 
   const int TP = std::max(1, std::min<int>(T, (int)std::max<uint32_t>(P, 1)));
-  // Chunks of both directions start at multiples of kFAlign / kBAlign
-  // elements; the gaps hold zero values (column / piece 0), and the arrays end
-  // with a chunk's worth of zeros.
+  // Backward chunks start at multiples of kBAlign elements; the gaps hold zero
+  // values (piece 0). Forward chunks have no gaps: an element of one would count
+  // as one of the last piece, and 0 times an infinite voxel is not 0. The arrays
+  // of both directions end with a chunk's worth of zeros.
   auto align_up = [](uint64_t x, uint64_t a) { return (x + a - 1) / a * a; };
   // ---- forward: every box's pieces (rows ascending) cut greedily into chunks
   // of at most kFChunkPieces pieces / kFChunkElems elements, the pieces of a
@@ -262,7 +263,7 @@ void build_host_panels(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_
         std::stable_sort(idx.begin() + i, idx.begin() + j, [&](uint32_t a, uint32_t b) {
           return rseg[a + 1] - rseg[a] > rseg[b + 1] - rseg[b];
         });
-        size += align_up(n, kFAlign);
+        size += n;
         i = j;
       }
       fsize[p] = size;
@@ -288,8 +289,7 @@ void build_host_panels(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_
       uint64_t e = fbase[p];
       uint32_t k = H.pfchunk[p];
       for (uint32_t i = 0, c = 0; i < np; ++i) {
-        if (c < fcut[p].size() && fcut[p][c] == i) {  // a chunk starts: align
-          e = fbase[p] + align_up(e - fbase[p], kFAlign);
+        if (c < fcut[p].size() && fcut[p][c] == i) {  // a chunk starts
           H.fchunk_piece[k++] = s0 + i;
           ++c;
         }
@@ -302,8 +302,7 @@ void build_host_panels(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_
       }
     }
   });
-  // a piece ends where the next one starts (the last of a chunk includes the
-  // zero gap before the next chunk)
+  // a piece ends where the next one starts
   H.fseg[nseg] = (uint32_t)nfel;
   H.fchunk_piece[H.pfchunk[P]] = (uint32_t)nseg;
 

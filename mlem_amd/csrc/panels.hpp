@@ -42,7 +42,7 @@ constexpr uint32_t kChunkPieces = 512;   // backward: pieces staged per chunk (a
 constexpr uint32_t kChunkElems = 8192;   // backward: elements staged per chunk (at most)
 constexpr uint32_t kFChunkPieces = 1024; // forward: pieces per chunk (at most)
 constexpr uint32_t kFChunkElems = 16384; // forward: elements per chunk (at most)
-constexpr uint32_t kFAlign = 4;          // forward chunks start at multiples of 4 elements
+constexpr uint32_t kFAlign = 1;          // forward chunks follow one another without gaps
 constexpr uint32_t kBAlign = 8;          // backward chunks start at multiples of 8 elements
 
 struct HostPanels {
@@ -56,8 +56,8 @@ struct HostPanels {
   std::vector<uint32_t> pseg;         // [npanels+1] first piece of each box
   std::vector<uint32_t> fseg;         // [nseg+1] first element of each piece
   std::vector<uint32_t> fslot;        // [nseg] row-major slot of each piece
-  std::vector<float> fval;            // values, piece-major, chunks aligned (zero gaps)
-  std::vector<uint16_t> fcol;         // column inside the piece's box (0 in the gaps)
+  std::vector<float> fval;            // values, piece-major, then a chunk of zeros
+  std::vector<uint16_t> fcol;         // column inside the piece's box
   std::vector<uint32_t> rowslot;      // [rows+1] first slot of each device row
   std::vector<uint32_t> pfchunk;      // [npanels+1] first forward chunk of each box
   std::vector<uint32_t> fchunk_piece; // [nfchunks+1] first piece of each forward chunk
