@@ -205,6 +205,8 @@ std::vector<uint32_t> nested_tiles(const std::vector<uint32_t>& ptr, uint32_t T,
       uint32_t e = s + 1;
       while (e < big[i + 1] && e - s < maxseg && (uint64_t)z + (ptr[e + 1] - ptr[s]) <= T) ++e;
       const uint32_t n = ptr[e] - ptr[s];
+      // the kernels hold T products, leading zeros included
+      if (n <= T && z + n > T) raise(MLEM_EINVAL, "a segment does not fit a nested tile");
       tiles.push_back(s);
       lead.push_back(n && n <= T ? z : 0);  // only tiles with stored elements
       s = e;
