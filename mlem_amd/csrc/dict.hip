@@ -3,18 +3,20 @@
 //
 // Every tile of at most T elements gets the sorted distinct indices it
 // gathers, and every element its 16-bit position among them. The tile's
-// indices are marked in a bitmap in LDS, one slab of 2^18 indices at a time;
-// a prefix sum of the words' population counts gives every marked index its
-// rank, which is its position. Slabs without an element are skipped.
+// indices are marked in a bitmap in LDS; a prefix sum of the words' population
+// counts gives every marked index its rank, which is its position. The bitmap
+// holds the pages that the tile uses, one after the other (a page: at most
+// 1/8192th of all indices, at least 32 of them), in slabs of 2^18 indices at a
+// time.
 //
 // What bounds it: the LDS passes over the slabs (clear, mark, count, look up;
-// about 1 us each for a 1024-lane workgroup, two of them per CU), 3 slabs per
-// forward tile of the 128x128x48 matrix and 6 per backward tile. It replaces a
-// bitonic sort of 8-byte keys in LDS (105 passes over a 128 KB array): both
-// projections' two passes 129 -> 4.9 ms on that matrix (168.5M elements), 600 ->
-// 40 ms on the 192x192x64 one (789.8M, 9 and 16 slabs). The sort would be
-// faster only where a tile's indices spread over more than about 800 slabs,
-// 2 * 10^8 rows or columns.
+// about 1 us each for a 1024-lane workgroup, two of them per CU).
+// Both projections' tiles of 2048 / 8192 / 16384 elements, allocation included, ms:
+//   192x192x64 voxels, 1.5M lines (282M elements)     20.6 / 10.8 / 9.7
+//   3M rows, 5M columns, 30M elements at random        7.8 /  7.5 / 8.6
+// A bitmap of all indices, without pages, took 41 / 17 / 16 and 14 / 33 / 34 (a
+// pass per slab that holds an element: up to one per element where the indices
+// spread far), a bitonic sort of 8-byte keys in LDS 43 / 110 / 222 and 8.9 / 27 / 89.
 #include <algorithm>
 #include <vector>
 
@@ -30,7 +32,7 @@ constexpr uint32_t kBuild = 1024;                 // lanes of a build workgroup
 constexpr uint32_t kSlabBits = 18;                // indices per bitmap slab (log2)
 constexpr uint32_t kWords = (1u << kSlabBits) / 32;
 constexpr uint32_t kLaneWords = kWords / kBuild;  // words counted by one lane
-constexpr uint32_t kMaxSlabs = 1u << (32 - kSlabBits);
+constexpr uint32_t kPages = 1u << 14;             // pages of all indices (at most)
 static_assert(kLaneWords == 8, "word() pads every lane's run of 8 words");
 
 // Word w of the bitmap: one word of padding after every 8, so that the lanes'
@@ -43,25 +45,26 @@ void check_launch(const char* what) {
 }
 
 // One tile per workgroup, at most EB elements per lane. Pass 1 (tiles4 ==
-// nullptr) counts the distinct indices of every tile; pass 2 writes the
+// nullptr) counts the distinct indices of every tile, and the runs of 32 indices
+// (128-byte lines of the gathered vector) that they lie in; pass 2 writes the
 // dictionary, padded with zeros to whole rounds of `nb` entries, and the
 // {value, position} element arrays, with the tile's leading zero elements and
-// padded with zeros to 64 elements. Indices
-// are below slab_words * 32 * 2^18.
+// padded with zeros to 64 elements. Indices are below kPages * 2^page_bits.
 template <uint32_t EB, int VK>
 __global__ __launch_bounds__(kBuild) void k_dict_rank(const uint2* __restrict__ el,
                                                       const uint2* __restrict__ tiles2,
                                                       const uint4* __restrict__ tiles4,
-                                                      uint32_t nb, uint32_t slab_words,
-                                                      uint32_t* __restrict__ nd_out,
+                                                      uint32_t nb, uint32_t page_bits,
+                                                      uint2* __restrict__ counts,
                                                       uint32_t* __restrict__ dict,
                                                       void* __restrict__ dval,
                                                       uint16_t* __restrict__ dlix) {
   constexpr uint32_t T = kBuild * EB;
   __shared__ uint32_t bits[kWords + kWords / 8];
   __shared__ uint16_t before[kWords + kWords / 8];  // marked indices before each word
-  __shared__ uint32_t slabs[kMaxSlabs / 32];        // slabs that hold an element
-  __shared__ uint32_t wsum[kBuild / kWave + 1];
+  __shared__ uint32_t pages[kPages / 32];           // pages that hold an element
+  __shared__ uint16_t pbefore[kPages / 32];         // such pages before each word
+  __shared__ uint32_t wsum[kBuild / kWave], lines;
   const uint32_t tile = blockIdx.x, t = threadIdx.x, lane = t % kWave, wave = t / kWave;
   uint32_t e0, e1, a0 = 0, lead = 0, g0 = 0;
   if (tiles4) {
@@ -77,73 +80,102 @@ __global__ __launch_bounds__(kBuild) void k_dict_rank(const uint2* __restrict__ 
   }
   const uint32_t count = e1 - e0;
   if (count > T || count == 0) {  // one long segment, or nothing: no dictionary
-    if (!tiles4 && t == 0) nd_out[tile] = 0;
+    if (!tiles4 && t == 0) counts[tile] = make_uint2(0, 0);
     return;
   }
+  // Sum over the lanes before this one; all: over all of them. A barrier lies
+  // between two calls.
+  auto scan = [&](uint32_t mine, uint32_t& all) __attribute__((always_inline)) {
+    uint32_t run = mine;  // inclusive sum over the wave
+#pragma unroll
+    for (uint32_t d = 1; d < kWave; d <<= 1) {
+      const uint32_t o = (uint32_t)__shfl_up((int)run, d);
+      if (lane >= d) run += o;
+    }
+    if (lane == kWave - 1) wsum[wave] = run;
+    __syncthreads();
+    uint32_t base = run - mine;
+    all = 0;
+    for (uint32_t w = 0; w < kBuild / kWave; ++w) {
+      const uint32_t v = wsum[w];
+      if (w < wave) base += v;
+      all += v;
+    }
+    return base;
+  };
   uint2 e[EB];
-  uint32_t pos[EB];
 #pragma unroll
   for (uint32_t j = 0; j < EB; ++j) e[j] = el[e0 + min(t + j * kBuild, count - 1)];
-  if (t < kMaxSlabs / 32) slabs[t] = 0;
+  if (t < kPages / 32) pages[t] = 0;
+  if (t == 0) lines = 0;
   __syncthreads();
 #pragma unroll
   for (uint32_t j = 0; j < EB; ++j) {
-    pos[j] = 0;
-    const uint32_t s = e[j].x >> kSlabBits;
-    if (!((slabs[s >> 5] >> (s & 31u)) & 1u)) atomicOr(&slabs[s >> 5], 1u << (s & 31u));
+    const uint32_t p = e[j].x >> page_bits;
+    if (!((pages[p >> 5] >> (p & 31u)) & 1u)) atomicOr(&pages[p >> 5], 1u << (p & 31u));
   }
   __syncthreads();
+  uint32_t used;  // pages
+  const uint32_t pb = scan(t < kPages / 32 ? __popc(pages[t]) : 0u, used);
+  if (t < kPages / 32) pbefore[t] = (uint16_t)pb;
+  __syncthreads();
+  uint32_t pos[EB];  // place in the used pages, then the index's rank
+#pragma unroll
+  for (uint32_t j = 0; j < EB; ++j) {
+    const uint32_t p = e[j].x >> page_bits, b = p & 31u;
+    const uint32_t at = pbefore[p >> 5] + __popc(pages[p >> 5] & ((1u << b) - 1u));
+    pos[j] = (at << page_bits) | (e[j].x & ((1u << page_bits) - 1u));
+  }
+  const uint64_t places = (uint64_t)used << page_bits;
+  const uint32_t slabs = (uint32_t)((places + (1u << kSlabBits) - 1) >> kSlabBits);
   uint32_t total = 0;  // distinct indices in the slabs so far (uniform)
-  for (uint32_t sw = 0; sw < slab_words; ++sw) {
-    for (uint32_t left = slabs[sw]; left; left &= left - 1) {  // uniform
-      const uint32_t s = sw * 32 + (uint32_t)__builtin_ctz(left);
-      for (uint32_t w = t; w < kWords + kWords / 8; w += kBuild) bits[w] = 0;
+  for (uint32_t s = 0; s < slabs; ++s) {
+    // words of the slab, to a whole lane's run
+    const uint64_t left = (places - ((uint64_t)s << kSlabBits) + 255) / 256 * 8;
+    const uint32_t words = (uint32_t)min(left, (uint64_t)kWords);
+    for (uint32_t w = t; w < words + words / 8; w += kBuild) bits[w] = 0;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < EB; ++j)
+      if (pos[j] >> kSlabBits == s)
+        atomicOr(&bits[word((pos[j] & ((1u << kSlabBits) - 1)) >> 5)], 1u << (pos[j] & 31u));
+    __syncthreads();
+    uint32_t mine = 0, full = 0;
+    if (t * kLaneWords < words) {
+#pragma unroll
+      for (uint32_t k = 0; k < kLaneWords; ++k) {
+        const uint32_t w = bits[word(t * kLaneWords + k)];
+        mine += __popc(w);
+        full += w != 0;
+      }
+    }
+    if (!tiles4 && full) atomicAdd(&lines, full);
+    uint32_t all;
+    uint32_t at = total + scan(mine, all);
+    total += all;
+    if (tiles4) {
+      if (t * kLaneWords < words) {
+#pragma unroll
+        for (uint32_t k = 0; k < kLaneWords; ++k) {
+          const uint32_t w = word(t * kLaneWords + k);
+          before[w] = (uint16_t)at;
+          at += __popc(bits[w]);
+        }
+      }
       __syncthreads();
 #pragma unroll
       for (uint32_t j = 0; j < EB; ++j)
-        if (e[j].x >> kSlabBits == s)
-          atomicOr(&bits[word((e[j].x & ((1u << kSlabBits) - 1)) >> 5)], 1u << (e[j].x & 31u));
-      __syncthreads();
-      uint32_t mine = 0;
-#pragma unroll
-      for (uint32_t k = 0; k < kLaneWords; ++k) mine += __popc(bits[word(t * kLaneWords + k)]);
-      uint32_t run = mine;  // inclusive sum over the wave
-#pragma unroll
-      for (uint32_t d = 1; d < kWave; d <<= 1) {
-        const uint32_t o = (uint32_t)__shfl_up((int)run, d);
-        if (lane >= d) run += o;
-      }
-      if (lane == kWave - 1) wsum[wave] = run;
-      __syncthreads();
-      uint32_t base = total, all = 0;
-      for (uint32_t w = 0; w < kBuild / kWave; ++w) {
-        const uint32_t v = wsum[w];
-        if (w < wave) base += v;
-        all += v;
-      }
-      uint32_t at = base + run - mine;
-#pragma unroll
-      for (uint32_t k = 0; k < kLaneWords; ++k) {
-        const uint32_t w = word(t * kLaneWords + k);
-        before[w] = (uint16_t)at;
-        at += __popc(bits[w]);
-      }
-      total += all;
-      __syncthreads();
-      if (tiles4) {
-#pragma unroll
-        for (uint32_t j = 0; j < EB; ++j)
-          if (e[j].x >> kSlabBits == s) {
-            const uint32_t w = word((e[j].x & ((1u << kSlabBits) - 1)) >> 5), b = e[j].x & 31u;
-            pos[j] = before[w] + __popc(bits[w] & ((1u << b) - 1u));
-            dict[g0 + pos[j]] = e[j].x;  // equal indices write the same word
-          }
-      }
-      __syncthreads();  // the next slab clears the bitmap
+        // (a rank is below 2^14: it is taken for a place of slab 0 at most)
+        if (pos[j] >> kSlabBits == s) {
+          const uint32_t w = word((pos[j] & ((1u << kSlabBits) - 1)) >> 5), b = pos[j] & 31u;
+          pos[j] = before[w] + __popc(bits[w] & ((1u << b) - 1u));
+          dict[g0 + pos[j]] = e[j].x;  // equal indices write the same word
+        }
     }
+    __syncthreads();  // the next slab clears the bitmap
   }
   if (!tiles4) {
-    if (t == 0) nd_out[tile] = total;
+    if (t == 0) counts[tile] = make_uint2(total, lines);
     return;
   }
   for (uint32_t i = total + t; i < (total + nb - 1) / nb * nb; i += kBuild) dict[g0 + i] = 0;
@@ -221,7 +253,8 @@ std::vector<uint32_t> nested_tiles(const std::vector<uint32_t>& ptr, uint32_t T,
 template <int NB, int EPT, int VK>
 void build_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, bool nested,
                 DictFormat& D, hipStream_t s) {
-  const uint32_t slab_words = (uint32_t)((((uint64_t)dim + (1u << kSlabBits) - 1) >> kSlabBits) + 31) / 32;
+  uint32_t page_bits = 5;
+  while (((uint64_t)kPages << page_bits) < dim) ++page_bits;
   constexpr uint32_t T = NB * EPT;
   static_assert(T % kBuild == 0, "build workgroups cover whole tiles");
   constexpr uint32_t EB = T / kBuild;  // elements per build lane
@@ -239,16 +272,16 @@ void build_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim,
     }
   } t2, ndb;
   MLEM_HIP(hipMalloc(&t2.p, sizeof(uint2) * d2.size()));
-  MLEM_HIP(hipMalloc(&ndb.p, 4ull * std::max<uint32_t>(nt, 1)));
+  MLEM_HIP(hipMalloc(&ndb.p, sizeof(uint2) * std::max<uint32_t>(nt, 1)));
   MLEM_HIP(hipMemcpyAsync(t2.p, d2.data(), sizeof(uint2) * d2.size(), hipMemcpyHostToDevice, s));
-  std::vector<uint32_t> nd(nt);
+  std::vector<uint2> nd(nt);
   if (nt) {
     hipLaunchKernelGGL((k_dict_rank<EB, VK>), dim3(nt), dim3(kBuild), 0, s, (const uint2*)el,
-                       (const uint2*)t2.p, (const uint4*)nullptr, (uint32_t)NB, slab_words,
-                       (uint32_t*)ndb.p,
+                       (const uint2*)t2.p, (const uint4*)nullptr, (uint32_t)NB, page_bits,
+                       (uint2*)ndb.p,
                        (uint32_t*)nullptr, (void*)nullptr, (uint16_t*)nullptr);
     check_launch("dictionary count launch");
-    MLEM_HIP(hipMemcpyAsync(nd.data(), ndb.p, 4ull * nt, hipMemcpyDeviceToHost, s));
+    MLEM_HIP(hipMemcpyAsync(nd.data(), ndb.p, sizeof(uint2) * nt, hipMemcpyDeviceToHost, s));
     MLEM_HIP(hipStreamSynchronize(s));
   }
   std::vector<uint4> d4(tl.size());
@@ -258,7 +291,7 @@ void build_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim,
     if (i == nt) break;
     const uint32_t count = ptr[tl[i + 1]] - ptr[tl[i]];
     if (count <= T) acc_a += (lead[i] + count + 63) / 64 * 64;
-    acc_g += (nd[i] + NB - 1) / NB * NB;  // whole rounds of one slot per wave
+    acc_g += (nd[i].x + NB - 1) / NB * NB;  // whole rounds of one slot per wave
   }
   if (acc_a + T > 0xFFFFFFFFull || acc_g > 0xFFFFFFFFull)
     raise(MLEM_EINVAL, "matrix too large for the dictionary format");
@@ -283,8 +316,8 @@ void build_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim,
   MLEM_HIP(hipMemcpyAsync(D.tiles, d4.data(), sizeof(uint4) * d4.size(), hipMemcpyHostToDevice, s));
   if (nt) {
     hipLaunchKernelGGL((k_dict_rank<EB, VK>), dim3(nt), dim3(kBuild), 0, s, (const uint2*)el,
-                       (const uint2*)nullptr, (const uint4*)D.tiles, (uint32_t)NB, slab_words,
-                       (uint32_t*)nullptr, D.dict, D.dval, D.dlix);
+                       (const uint2*)nullptr, (const uint4*)D.tiles, (uint32_t)NB, page_bits,
+                       (uint2*)nullptr, D.dict, D.dval, D.dlix);
     check_launch("dictionary fill launch");
   }
   const uint64_t per = kBlock / kWave;
