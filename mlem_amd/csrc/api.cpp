@@ -221,27 +221,46 @@ GroupLaunch named_launch(int kind, int param, const GroupLaunch& open) {
 // tiles run by 512-lane blocks, two per CU (LDS- and register-bound), are the
 // fastest once every CU gets several: pet (168.4M elements) forward / backward
 // 224 / 218 us against 250 / 246 with 8192. A small matrix is bound by the
-// latency of one tile and by its last wave of tiles (us, 16384 / 8192 / 2048
-// elements, launch included):
-//   29.5M elements  50.3 / 54.2 / 64.1 forward, 44.3 / 45.2 / 60.3 backward
-//   25.4M           41.3 / 41.7 / 44.4,          41.9 / 43.4 / 61.8
-//    9.7M           23.2 / 20.8 / 21.1,          23.0 / 22.2 / 30.2
-//    3.7M           13.2 / 12.2 / 12.2,          13.0 / 11.7 / 12.8
-//    1.9M           12.4 / 10.1 /  9.3,          12.2 /  9.5 /  9.1
-//    0.5M           11.4 /  9.5 /  7.7,          10.7 /  9.0 /  6.9
-// A segment longer than a tile is summed with direct gathers (EXACT: by one
-// lane), so tiles hold the longest segment where the largest ones can.
+// latency of one tile and by its last wave of tiles (us of one FAST product, launch
+// included, 16384 / 8192 / 2048 elements):
+//   lines of response  9.2M elements  23.6 / 22.0 / 22.0 forward, 21.6 / 20.8 / 22.8 backward
+//                      4.9M           17.5 / 14.9 / 15.0,         15.9 / 14.2 / 14.1
+//                      2.4M           12.8 / 11.2 / 10.2,         12.0 / 11.0 / 10.2
+//                      0.4M           11.0 /  9.0 /  7.5,         11.0 /  8.3 /  6.6
+// but gathers more lines in all, as a line is gathered once per tile that needs
+// it: about 9 us per million lines, which is what it gains at a quarter of a million
+//   lines of response 15.2M, 0.3M lines more  31.1 / 33.4 (8192), 28.9 / 30.2
+//   random           18.0M, 3.5M              64.8 / 80.0,        62.0 / 76.0
+//   random           12.0M, 1.4M              29.7 / 37.5,        28.3 / 36.8
+//   random            2.2M, 0.8M              13.3 / 14.1 (2048), 13.3 / 13.6
+// And a tile of few segments keeps few lanes busy; where tiles wait for a place
+// as well, smaller ones that hold one long segment take longer: 11x12x12 voxels,
+// 6.6M elements, backward 44.6 / 57.8 FAST and 99.7 / 136.6 EXACT (8192); 5000
+// columns of 400 elements 16.4 / 20.1 EXACT (2048). A segment longer than a tile is
+// summed with direct gathers (EXACT: by one lane), so tiles hold the longest
+// segment where the largest ones can.
 // mlem_autotune measures the alternatives on the real matrix.
-GroupLaunch default_launch(uint64_t nnz, const std::vector<uint32_t>& ptr) {
+GroupLaunch default_launch(uint64_t nnz, const std::vector<uint32_t>& ptr, const uint2* el,
+                           uint32_t dim, hipStream_t s) {
+  constexpr double kMoreLines = 250000.0;
+  GroupLaunch g = make_launch(kDictWide, 32);  // the same FAST sums with every tile size
+  if (nnz > 20000000 || nnz == 0 || !el) return g;
   uint32_t longest = 0;
-  if (nnz <= 20000000)
-    for (size_t i = 0; i + 1 < ptr.size(); ++i) longest = std::max(longest, ptr[i + 1] - ptr[i]);
-  GroupLaunch g = make_launch(kDictWide, 32);
-  if (nnz <= 2500000 && longest + 3 <= 256 * 8)
+  double squares = 0.0;
+  for (size_t i = 0; i + 1 < ptr.size(); ++i) {
+    const uint32_t n = ptr[i + 1] - ptr[i];
+    longest = std::max(longest, n);
+    squares += (double)n * n;
+  }
+  const double length = squares / (double)nnz;  // of an element's segment, on average
+  if (longest + 3 > 512 * 16 || (nnz > 2500000 && length > 512 * 16 / 5)) return g;
+  const std::array<double, 3> lines = tile_lines(ptr, el, dim, s);
+  if (lines[1] - lines[0] > kMoreLines) return g;
+  g = make_launch(kDictWide, 16);
+  if (nnz <= 2500000 && longest + 3 <= 256 * 8 && length <= 256 * 8 / 5 &&
+      lines[2] - lines[1] <= kMoreLines)
     g = make_launch(kDict, 8);
-  else if (nnz <= 20000000 && longest + 3 <= 512 * 16)
-    g = make_launch(kDictWide, 16);
-  g.nested = g.kind != kDictWide || g.ept != 32;  // the same FAST sums with every tile size
+  g.nested = true;
   return g;
 }
 
@@ -374,8 +393,8 @@ void finish_open(mlem_matrix* h, unsigned flags) {
 
   const double avgRow = m.rows ? (double)m.nnz / m.rows : 1.0;
   download_pointers(m, m.stream);
-  m.fwd = m.fwd_open = default_launch(m.nnz, m.h_rowptr);
-  m.bwd = m.bwd_open = default_launch(m.nnz, m.h_colptr);
+  m.fwd = m.fwd_open = default_launch(m.nnz, m.h_rowptr, m.csr, m.cols, m.stream);
+  m.bwd = m.bwd_open = default_launch(m.nnz, m.h_colptr, m.csc, m.rows, m.stream);
   m.scatter = make_launch(kGroups, lanes_for(avgRow));
   prepare_tiles(m, m.stream);
   if (env_int("MLEM_AUTOTUNE", 0) > 0) autotune(m);

@@ -18,6 +18,7 @@
 // pass per slab that holds an element: up to one per element where the indices
 // spread far), a bitonic sort of 8-byte keys in LDS 43 / 110 / 222 and 8.9 / 27 / 89.
 #include <algorithm>
+#include <array>
 #include <vector>
 
 #include "internal.hpp"
@@ -223,28 +224,42 @@ __global__ __launch_bounds__(kBlock) void k_dict_pack(uint32_t* __restrict__ dic
   if (l == 0) meta[s] = base | (wide ? 0x80000000u : 0u);
 }
 
-// Tiles of at most T elements, leading zeros included, and `maxseg` segments
-// inside the tiles of 16384 elements and 512 segments (DictFormat). A larger
-// tile that is one long segment stays whole.
+// Cuts the segments [s0, s1) of one tile of 16384 elements and 512 segments into
+// tiles of at most T elements, leading zeros included, and `maxseg` segments
+// (DictFormat): tile(first, end, leading zeros). A larger segment stays whole.
+template <class Tile>
+void cut_nested(const std::vector<uint32_t>& ptr, uint32_t s0, uint32_t s1, uint32_t T,
+                uint32_t maxseg, Tile&& tile) {
+  for (uint32_t s = s0, e; s < s1; s = e) {
+    const uint32_t z = (ptr[s] - ptr[s0]) & 3u;
+    e = s + 1;
+    while (e < s1 && e - s < maxseg && (uint64_t)z + (ptr[e + 1] - ptr[s]) <= T) ++e;
+    tile(s, e, z);
+  }
+}
+
 std::vector<uint32_t> nested_tiles(const std::vector<uint32_t>& ptr, uint32_t T, uint32_t maxseg,
                                    std::vector<uint32_t>& lead) {
   const std::vector<uint32_t> big = partition_tiles(ptr, 16384, 512);
   std::vector<uint32_t> tiles;
   lead.clear();
   for (size_t i = 0; i + 1 < big.size(); ++i)
-    for (uint32_t s = big[i]; s < big[i + 1];) {
-      const uint32_t z = (ptr[s] - ptr[big[i]]) & 3u;
-      uint32_t e = s + 1;
-      while (e < big[i + 1] && e - s < maxseg && (uint64_t)z + (ptr[e + 1] - ptr[s]) <= T) ++e;
+    cut_nested(ptr, big[i], big[i + 1], T, maxseg, [&](uint32_t s, uint32_t e, uint32_t z) {
       const uint32_t n = ptr[e] - ptr[s];
       // the kernels hold T products, leading zeros included
       if (n <= T && z + n > T) raise(MLEM_EINVAL, "a segment does not fit a nested tile");
       tiles.push_back(s);
       lead.push_back(n && n <= T ? z : 0);  // only tiles with stored elements
-      s = e;
-    }
+    });
   tiles.push_back((uint32_t)ptr.size() - 1);
   return tiles;
+}
+
+// Pages of at least 32 indices that cover dim of them.
+uint32_t page_bits_for(uint32_t dim) {
+  uint32_t b = 5;
+  while (((uint64_t)kPages << b) < dim) ++b;
+  return b;
 }
 
 // Build the dictionary format of one projection from its device-order
@@ -253,8 +268,7 @@ std::vector<uint32_t> nested_tiles(const std::vector<uint32_t>& ptr, uint32_t T,
 template <int NB, int EPT, int VK>
 void build_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, bool nested,
                 DictFormat& D, hipStream_t s) {
-  uint32_t page_bits = 5;
-  while (((uint64_t)kPages << page_bits) < dim) ++page_bits;
+  const uint32_t page_bits = page_bits_for(dim);
   constexpr uint32_t T = NB * EPT;
   static_assert(T % kBuild == 0, "build workgroups cover whole tiles");
   constexpr uint32_t EB = T / kBuild;  // elements per build lane
@@ -372,6 +386,55 @@ std::vector<uint32_t> partition_tiles(const std::vector<uint32_t>& ptr, uint32_t
     s = e;
   }
   return tiles;
+}
+
+std::array<double, 3> tile_lines(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim,
+                                 hipStream_t s) {
+  constexpr uint32_t kSample = 64, T[3] = {16384, 8192, 2048}, kSeg[3] = {512, 512, 256};
+  const uint32_t n = (uint32_t)ptr.size() - 1;
+  // the tiles of every size in the sampled large ones, one after the other: a
+  // range of elements from each entry to the next, those in which `size` is set
+  std::vector<uint2> range;
+  std::vector<int> size;
+  uint64_t covered = 0;
+  for (uint32_t i = 0, s0 = 0, s1 = 0; i < kSample && s1 < n; ++i) {
+    s0 = std::max(s1, (uint32_t)((uint64_t)n * i / kSample));
+    s1 = s0 + 1;
+    while (s1 < n && s1 - s0 < kSeg[0] && ptr[s1 + 1] - ptr[s0] <= T[0]) ++s1;
+    covered += ptr[s1] - ptr[s0];
+    for (int k = 0; k < 3; ++k) {
+      cut_nested(ptr, s0, s1, T[k], kSeg[k], [&](uint32_t b, uint32_t, uint32_t) {
+        range.push_back(make_uint2(b, ptr[b]));
+        size.push_back(k);
+      });
+      range.push_back(make_uint2(s1, ptr[s1]));
+      size.push_back(-1);
+    }
+  }
+  std::array<double, 3> lines{0.0, 0.0, 0.0};
+  if (range.size() < 2 || covered == 0) return lines;
+  struct Buf {
+    void* p = nullptr;
+    ~Buf() {
+      if (p) (void)hipFree(p);
+    }
+  } buf;
+  std::vector<uint2> counts(range.size() - 1);
+  MLEM_HIP(hipMalloc(&buf.p, 2 * sizeof(uint2) * range.size()));
+  uint2 *d_range = static_cast<uint2*>(buf.p), *d_counts = d_range + range.size();
+  MLEM_HIP(hipMemcpyAsync(d_range, range.data(), sizeof(uint2) * range.size(),
+                          hipMemcpyHostToDevice, s));
+  hipLaunchKernelGGL((k_dict_rank<16, kF32>), dim3((unsigned)counts.size()), dim3(kBuild), 0, s, el,
+                     (const uint2*)d_range, (const uint4*)nullptr, 0u, page_bits_for(dim), d_counts,
+                     (uint32_t*)nullptr, (void*)nullptr, (uint16_t*)nullptr);
+  check_launch("tile sample launch");
+  MLEM_HIP(hipMemcpyAsync(counts.data(), d_counts, sizeof(uint2) * counts.size(),
+                          hipMemcpyDeviceToHost, s));
+  MLEM_HIP(hipStreamSynchronize(s));
+  for (size_t i = 0; i < counts.size(); ++i)
+    if (size[i] >= 0) lines[(size_t)size[i]] += counts[i].y;
+  for (double& l : lines) l *= (double)ptr[n] / (double)covered;
+  return lines;
 }
 
 void ensure_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, int nb, int ept,
