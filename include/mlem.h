@@ -136,7 +136,8 @@ MLEM_API int mlem_open_host(uint32_t rows, uint32_t cols, uint64_t nnz,
  * backprojection their CSC parts over PCIe through two device buffers, the
  * copy of one block overlapping the kernels of the block before. The CSR parts
  * of blocks of 2^20 elements or more cross PCIe packed (without loss: about 5
- * of 8 bytes per element where columns advance by few different steps) and are
+ * of 8 bytes per element where columns advance by few different steps; blocks
+ * that a sample expects to shrink by less than a tenth stay as they are) and are
  * unpacked into a third buffer, if the device has room for it at open. A
  * reconstruction iteration streams each CSR part once and builds the block's
  * CSC on the device right after its forward projection (mlem_stream_passes).

@@ -29,86 +29,119 @@ uint64_t align16(uint64_t n) { return (n + 15) & ~15ull; }
 // with 32-bit offsets.
 constexpr uint64_t kMaxBlockNnz = (1ull << 32) - 1024;
 
-uint64_t pack_chunks(uint64_t nnz) { return (nnz + kPackChunk - 1) / kPackChunk; }
+uint64_t pack_chunks_of(uint64_t nnz) { return (nnz + kPackChunk - 1) / kPackChunk; }
 // Bytes between a packed part's row pointers and its first chunk.
-uint64_t pack_front(uint64_t nnz) { return sizeof(PackHead) * pack_chunks(nnz) + 4 * kPackTable; }
+uint64_t pack_front(uint64_t nnz) { return sizeof(PackHead) * pack_chunks_of(nnz) + 4 * kPackTable; }
+
+uint32_t step_hash(uint32_t d) { return d * 2654435761u; }
 
 // The steps between neighbouring elements' columns that get a code: the most
-// frequent of a sample of 16 chunks.
-void pack_table(const uint2* el, uint64_t nnz, uint32_t* table) {
-  std::vector<uint32_t> d;
-  const uint64_t n = pack_chunks(nnz), every = std::max<uint64_t>(1, n / 16);
-  for (uint64_t c = 0; c < n; c += every) {
-    const uint64_t e = std::min(nnz, (c + 1) * kPackChunk);
-    for (uint64_t k = c * kPackChunk + 1; k < e; ++k) d.push_back(el[k].x - el[k - 1].x);
+// frequent of a sample of 16 chunks, counted in a hash table. pays: whether a block
+// packed with them is expected to be at least a tenth smaller (7.25 of 8 bytes an
+// element): else the copies would gain less than the packing costs at open.
+struct PackSteps {
+  uint32_t step[kPackTable];
+  bool pays = false;
+};
+PackSteps pack_steps(const ElementFetch& fetch, uint64_t base, uint64_t nnz) {
+  constexpr uint64_t kRuns = 16;
+  constexpr uint32_t kBits = 17;  // twice the steps of the sample
+  PackSteps t;
+  std::vector<uint2> el(kPackChunk + 1), count(1u << kBits, make_uint2(0, 0));  // {step, times}
+  uint64_t total = 0;
+  for (uint64_t i = 0; i < kRuns; ++i) {
+    const uint64_t at = nnz * i / kRuns, n = std::min<uint64_t>(el.size(), nnz - at);
+    fetch(el.data(), base + at, n);
+    for (uint64_t k = 1; k < n; ++k) {
+      const uint32_t d = el[k].x - el[k - 1].x;
+      uint32_t h = step_hash(d) >> (32 - kBits);
+      while (count[h].y && count[h].x != d) h = (h + 1) & ((1u << kBits) - 1);
+      count[h].x = d;
+      ++count[h].y;
+      ++total;
+    }
   }
-  std::sort(d.begin(), d.end());
   std::vector<std::pair<uint32_t, uint32_t>> runs;  // {times, step}
-  for (size_t i = 0; i < d.size();) {
-    size_t j = i;
-    while (j < d.size() && d[j] == d[i]) ++j;
-    runs.emplace_back((uint32_t)(j - i), d[i]);
-    i = j;
-  }
-  std::sort(runs.begin(), runs.end(), [](const auto& a, const auto& b) {
-    return a.first != b.first ? a.first > b.first : a.second < b.second;
-  });
+  for (const uint2& c : count)
+    if (c.y) runs.emplace_back(c.y, c.x);
   const size_t k = std::min<size_t>(runs.size(), kPackEscape);
-  for (size_t i = 0; i < kPackTable; ++i) table[i] = k ? runs[std::min(i, k - 1)].second : 0;
+  std::partial_sort(runs.begin(), runs.begin() + (std::ptrdiff_t)k, runs.end(),
+                    [](const auto& a, const auto& b) {
+                      return a.first != b.first ? a.first > b.first : a.second < b.second;
+                    });
+  uint64_t coded = 0;
+  for (size_t i = 0; i < k; ++i) coded += runs[i].first;
+  t.pays = total && 4.0 + 1.0 + 4.0 * (double)(total - coded) / (double)total <= 7.25;
+  for (size_t i = 0; i < kPackTable; ++i) t.step[i] = k ? runs[std::min(i, k - 1)].second : 0;
+  return t;
 }
 
-// Packs the nnz elements at front + pack_front(nnz) in place (a chunk never grows,
-// so its packed form ends before the next chunk's elements). Returns the end of
-// the packed part.
-char* pack_block(char* front, uint64_t nnz) {
+// Packs chunks c0 .. c1-1 of the nnz elements at front + pack_front(nnz) in place,
+// from the place of chunk c0's elements on (a chunk never grows, so its packed
+// form ends before the next chunk's elements). Returns the end of the packed chunks.
+char* pack_chunks(char* front, uint64_t nnz, uint64_t c0, uint64_t c1, const PackSteps& t) {
   PackHead* heads = reinterpret_cast<PackHead*>(front);
-  uint32_t* table = reinterpret_cast<uint32_t*>(heads + pack_chunks(nnz));
   char* const first = front + pack_front(nnz);
   const uint2* el = reinterpret_cast<const uint2*>(first);
-  pack_table(el, nnz, table);
   constexpr uint32_t kSlots = 1024;  // open addressing: step -> code
-  std::vector<uint32_t> key(kSlots), code(kSlots, kPackEscape);
-  auto slot = [](uint32_t d) { return (d * 2654435761u) >> 22; };
+  struct Slot {
+    uint32_t step = 0, code = kPackEscape;
+  };
+  std::vector<Slot> slots(kSlots);
+  auto find = [&](uint32_t d) {
+    uint32_t h = step_hash(d) >> 22;
+    while (slots[h].code != kPackEscape && slots[h].step != d) h = (h + 1) % kSlots;
+    return h;
+  };
   for (uint32_t c = 0; c < kPackEscape; ++c) {
-    uint32_t h = slot(table[c]);
-    while (code[h] != kPackEscape && key[h] != table[c]) h = (h + 1) % kSlots;
-    if (code[h] != kPackEscape) continue;  // the table's filling
-    key[h] = table[c];
-    code[h] = c;
+    Slot& e = slots[find(t.step[c])];
+    if (e.code == kPackEscape) e = Slot{t.step[c], c};  // (else the table's filling)
   }
-  std::vector<uint2> raw(kPackChunk);
   std::vector<uint8_t> codes(kPackChunk);
   std::vector<uint32_t> steps(kPackChunk);
-  char* out = first;
-  for (uint64_t c = 0; c < pack_chunks(nnz); ++c) {
+  char* out = first + 8ull * kPackChunk * c0;
+  for (uint64_t c = c0; c < c1; ++c) {
     const uint32_t m = (uint32_t)std::min<uint64_t>(kPackChunk, nnz - c * kPackChunk);
-    std::copy(el + c * kPackChunk, el + c * kPackChunk + m, raw.begin());
+    const uint2* raw = el + c * kPackChunk;  // at `out` or beyond
     uint32_t prev = 0, ns = 0;
     for (uint32_t k = 0; k < m; ++k) {
       const uint32_t d = raw[k].x - prev;
       prev = raw[k].x;
-      uint32_t h = slot(d);
-      while (code[h] != kPackEscape && key[h] != d) h = (h + 1) % kSlots;
-      codes[k] = (uint8_t)code[h];
+      const uint32_t code = slots[find(d)].code;
+      codes[k] = (uint8_t)code;
       steps[ns] = d;
-      ns += code[h] == kPackEscape;
+      ns += code == kPackEscape;
     }
     std::fill(codes.begin() + m, codes.end(), (uint8_t)0);
     const uint64_t vb = align16(4ull * m), cb = align16(m), bytes = vb + cb + align16(4ull * ns);
     const bool keep = bytes >= 8ull * m;
     heads[c] = PackHead{(uint32_t)((out - first) / 16), m, keep ? kPackRaw : ns, 0};
     if (keep) {
-      std::memcpy(out, raw.data(), 8ull * m);
+      std::memmove(out, raw, 8ull * m);
       out += align16(8ull * m);
       continue;
     }
     uint32_t* v = reinterpret_cast<uint32_t*>(out);
-    for (uint32_t k = 0; k < m; ++k) v[k] = raw[k].y;
+    for (uint32_t k = 0; k < m; ++k) v[k] = raw[k].y;  // (reads run ahead of the writes)
     std::memcpy(out + vb, codes.data(), cb);
     std::memcpy(out + vb + cb, steps.data(), 4ull * ns);
     out += bytes;
   }
   return out;
+}
+
+// work(0) .. work(n - 1) on threads of their own, as far as there are any.
+template <class Work>
+void on_threads(unsigned n, Work&& work) {
+  std::vector<std::thread> pool;
+  unsigned t = 1;
+  try {
+    for (; t < n; ++t) pool.emplace_back(work, t);
+  } catch (const std::exception&) {  // no more threads: this one does the rest
+  }
+  work(0);
+  for (; t < n; ++t) work(t);
+  for (auto& th : pool) th.join();
 }
 
 }  // namespace
@@ -164,33 +197,43 @@ StreamedMatrix* build_streamed(uint32_t rows, uint32_t cols, uint64_t nnz,
     }
     B.rows = r - r0;
     B.nnz = n;
-    B.csr_off = off;
     B.csr_bytes = align16(4ull * ((uint64_t)B.rows + 1)) + 8 * n;
-    off += align16(B.csr_bytes + pack_front(n));
-    B.csc_off = off;
     B.csc_bytes = colpart + 8 * n;
-    off += align16(B.csc_bytes);
     S->blocks.push_back(B);
     if (rows == 0) break;
     r0 = r;
   }
+
+  // Blocks kept in device memory: the first ones whose two parts fit the
+  // resident budget; only the others are streamed. Of these, the larger ones may
+  // be packed and get room for the chunks' heads and the table of steps.
+  uint64_t kept = 0, streamed_part = 0;
+  std::vector<char> keep(S->blocks.size(), 0), room(S->blocks.size(), 0);
+  for (size_t b = 0; b < S->blocks.size(); ++b) {
+    StreamBlock& B = S->blocks[b];
+    const uint64_t both = align16(B.csr_bytes) + B.csc_bytes;
+    keep[b] = kept + both <= resident_bytes && streamed_part == 0;
+    room[b] = !keep[b] && B.nnz >= kPackMin;
+    const uint64_t csr = room[b] ? B.csr_bytes + pack_front(B.nnz) + 16 : B.csr_bytes;
+    if (keep[b]) {
+      kept += both;
+    } else {
+      streamed_part = std::max(streamed_part, std::max(csr, B.csc_bytes));
+      S->max_stream_nnz = std::max(S->max_stream_nnz, B.nnz);
+    }
+    B.csr_off = off;
+    off += align16(csr);
+    B.csc_off = off;
+    off += align16(B.csc_bytes);
+  }
   S->host_bytes = std::max<uint64_t>(off, 16);
   MLEM_HIP(hipHostMalloc((void**)&S->host, S->host_bytes, hipHostMallocDefault));
 
-  // Blocks kept in device memory: the first ones whose two parts fit the
-  // resident budget; only the others are streamed.
-  uint64_t kept = 0, streamed_part = 0;
-  for (StreamBlock& B : S->blocks) {
-    const uint64_t both = align16(B.csr_bytes) + B.csc_bytes;
-    if (kept + both <= resident_bytes && streamed_part == 0) {
-      MLEM_HIP(hipMalloc((void**)&B.resident, both));
-      kept += both;
-    } else {
-      const uint64_t packed = B.csr_bytes + pack_front(B.nnz) + 16;
-      streamed_part = std::max(streamed_part, std::max(packed, B.csc_bytes));
-      S->max_stream_nnz = std::max(S->max_stream_nnz, B.nnz);
+  for (size_t b = 0; b < S->blocks.size(); ++b)
+    if (keep[b]) {
+      StreamBlock& B = S->blocks[b];
+      MLEM_HIP(hipMalloc((void**)&B.resident, align16(B.csr_bytes) + B.csc_bytes));
     }
-  }
   S->part_bytes = streamed_part;
   for (int i = 0; i < 2; ++i) {
     MLEM_HIP(hipMalloc((void**)&S->dev[i], std::max<uint64_t>(S->part_bytes, 16)));
@@ -223,16 +266,16 @@ StreamedMatrix* build_streamed(uint32_t rows, uint32_t cols, uint64_t nnz,
 
   // Fill the blocks in parallel: CSR part from the source, CSC part by a
   // counting sort over the block's columns (rows ascending in every column).
-  const unsigned nthreads = (unsigned)std::max<size_t>(
-      1, std::min<size_t>({S->blocks.size(), 16, std::max(1u, std::thread::hardware_concurrency())}));
+  const unsigned hw = std::min(16u, std::max(1u, std::thread::hardware_concurrency()));
+  const unsigned nthreads = (unsigned)std::max<size_t>(1, std::min<size_t>(S->blocks.size(), hw));
   std::atomic<uint64_t> bad{0};
-  std::vector<std::string> errors(nthreads);
+  std::vector<std::string> errors(hw);
+  std::vector<PackSteps> steps(S->blocks.size());
   auto work = [&](unsigned tid) {
     try {
       std::vector<uint32_t> next(cols);
       for (size_t b = tid; b < S->blocks.size(); b += nthreads) {
         StreamBlock& B = S->blocks[b];
-        const bool pack = S->expand && !B.resident && B.nnz >= kPackMin;
         char* csr = S->host + B.csr_off;
         char* csc = S->host + B.csc_off;
         uint32_t* rp = reinterpret_cast<uint32_t*>(csr);
@@ -240,7 +283,8 @@ StreamedMatrix* build_streamed(uint32_t rows, uint32_t cols, uint64_t nnz,
         rp[0] = 0;
         for (uint32_t k = 0; k < B.rows; ++k) rp[k + 1] = (uint32_t)(rowidx[B.row0 + k] - base);
         char* front = csr + align16(4ull * ((uint64_t)B.rows + 1));
-        uint2* el = reinterpret_cast<uint2*>(front + (pack ? pack_front(B.nnz) : 0));
+        if (S->expand && room[b]) steps[b] = pack_steps(fetch, base, B.nnz);
+        uint2* el = reinterpret_cast<uint2*>(front + (steps[b].pays ? pack_front(B.nnz) : 0));
         if (B.nnz) fetch(el, base, B.nnz);
         uint32_t* cp = reinterpret_cast<uint32_t*>(csc);
         std::fill(cp, cp + (uint64_t)cols + 1, 0u);
@@ -261,7 +305,6 @@ StreamedMatrix* build_streamed(uint32_t rows, uint32_t cols, uint64_t nnz,
         for (uint32_t k = 0; k < B.rows; ++k)
           for (uint32_t e = rp[k]; e < rp[k + 1]; ++e)
             ce[next[el[e].x]++] = make_uint2(B.row0 + k, el[e].y);
-        if (pack) B.packed_bytes = (uint64_t)(pack_block(front, B.nnz) - csr);
       }
     } catch (const ApiError& e) {
       errors[tid] = e.msg;
@@ -269,15 +312,61 @@ StreamedMatrix* build_streamed(uint32_t rows, uint32_t cols, uint64_t nnz,
       errors[tid] = e.what();
     }
   };
-  std::vector<std::thread> pool;
-  for (unsigned t = 1; t < nthreads; ++t) pool.emplace_back(work, t);
-  work(0);
-  for (auto& t : pool) t.join();
-  for (const std::string& e : errors)
-    if (!e.empty()) raise(MLEM_EIO, e);
-  if (bad)
-    raise(MLEM_EFORMAT, std::to_string(bad.load()) + " matrix elements have a column index >= " +
-                            std::to_string(cols));
+  auto check = [&] {
+    for (const std::string& e : errors)
+      if (!e.empty()) raise(MLEM_EIO, e);
+    if (bad)
+      raise(MLEM_EFORMAT, std::to_string(bad.load()) + " matrix elements have a column index >= " +
+                              std::to_string(cols));
+  };
+  on_threads(nthreads, work);
+  check();
+
+  // Pack: a matrix of few blocks has each cut into groups of chunks, so that more
+  // threads have some (about 1 ns an element on one thread: 67M elements in one
+  // block 75 ms, opened in 690). The groups keep their places, so every one is a
+  // copy of its own, and those cost about 9 us each: at most four.
+  struct Group {
+    size_t block;
+    uint64_t c0, c1;
+  };
+  std::vector<Group> groups;
+  for (size_t b = 0; b < S->blocks.size(); ++b) {
+    StreamBlock& B = S->blocks[b];
+    if (!steps[b].pays) continue;
+    const uint64_t n = pack_chunks_of(B.nnz);
+    const uint64_t g = std::max<uint64_t>(
+        1, std::min<uint64_t>({hw / S->blocks.size(), B.nnz / kPackMin, 4}));
+    B.packed.resize(g);
+    for (uint64_t i = 0; i < g; ++i) groups.push_back(Group{b, n * i / g, n * (i + 1) / g});
+    char* front = S->host + B.csr_off + align16(4ull * ((uint64_t)B.rows + 1));
+    std::memcpy(front + sizeof(PackHead) * n, steps[b].step, sizeof(steps[b].step));
+  }
+  std::atomic<size_t> next_group{0};
+  auto pack = [&](unsigned tid) {
+    try {
+      for (size_t i; (i = next_group++) < groups.size();) {
+        const Group& G = groups[i];
+        StreamBlock& B = S->blocks[G.block];
+        char* csr = S->host + B.csr_off;
+        char* front = csr + align16(4ull * ((uint64_t)B.rows + 1));
+        char* begin = G.c0 ? front + pack_front(B.nnz) + 8ull * kPackChunk * G.c0 : csr;
+        char* end = pack_chunks(front, B.nnz, G.c0, G.c1, steps[G.block]);
+        size_t at = 0;  // of this group among its block's
+        while (i > at && groups[i - at - 1].block == G.block) ++at;
+        B.packed[at] = {(uint64_t)(begin - csr), (uint64_t)(end - begin)};
+      }
+    } catch (const std::exception& e) {
+      errors[tid] = e.what();
+    }
+  };
+  if (!groups.empty()) {
+    on_threads((unsigned)std::min<size_t>(groups.size(), hw), pack);
+    check();
+  } else if (S->expand) {  // nothing to unpack
+    MLEM_HIP(hipFree(S->expand));
+    S->expand = nullptr;
+  }
 
   for (StreamBlock& B : S->blocks)
     if (B.resident) {
@@ -325,11 +414,16 @@ void stream_pass(const DevMatrix& m, bool csc, K&& kernel, hipStream_t s) {
       continue;
     }
     const int i = (int)(n_streamed++ & 1);
-    const bool packed = !csc && B.packed_bytes;
-    const uint64_t off = csc ? B.csc_off : B.csr_off;
-    const uint64_t n = csc ? B.csc_bytes : packed ? B.packed_bytes : B.csr_bytes;
+    const bool packed = !csc && !B.packed.empty();
     MLEM_HIP(hipStreamWaitEvent(S.copy, S.freed[i], 0));
-    MLEM_HIP(hipMemcpyAsync(S.dev[i], S.host + off, n, hipMemcpyHostToDevice, S.copy));
+    if (packed) {
+      for (const StreamBlock::Range& g : B.packed)
+        MLEM_HIP(hipMemcpyAsync(S.dev[i] + g.at, S.host + B.csr_off + g.at, g.bytes,
+                                hipMemcpyHostToDevice, S.copy));
+    } else {
+      MLEM_HIP(hipMemcpyAsync(S.dev[i], S.host + (csc ? B.csc_off : B.csr_off),
+                              csc ? B.csc_bytes : B.csr_bytes, hipMemcpyHostToDevice, S.copy));
+    }
     MLEM_HIP(hipEventRecord(S.copied[i], S.copy));
     MLEM_HIP(hipStreamWaitEvent(s, S.copied[i], 0));
     const uint2* el = reinterpret_cast<const uint2*>(S.dev[i] + pointers);
