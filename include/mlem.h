@@ -273,7 +273,7 @@ MLEM_API int mlem_reconstruct(mlem_matrix* m, const int32_t* y, uint32_t rows,
  * before the call. With both statistics arrays NULL the call only enqueues
  * (no synchronization; it can be captured into a HIP graph), otherwise it
  * returns when done. Its scratch (device-order copies of y and x, the ratio
- * vector, FP64 statistics partials) is one static 64 MiB device array per
+ * vector, FP64 statistics partials) is one static 65 MiB device array per
  * GPU, shared by every call on that GPU: calls that overlap on one GPU race.
  * Matrices that need more scratch (4 * (2 rows + cols) bytes plus the
  * statistics) get MLEM_EINVAL; streamed matrices are not supported. */

@@ -22,7 +22,10 @@ using namespace mlem;
 
 namespace {
 
-constexpr size_t kScratchBytes = 64ull << 20;  // 64 MiB per GPU
+// 65 MiB per GPU: 64 for the vectors, and the statistics partials (16 bytes a tile)
+// of the smallest dictionary tiles that a matrix of that size is opened with, up
+// to 0.9 MB.
+constexpr size_t kScratchBytes = 65ull << 20;
 constexpr unsigned kRing = 1024;               // statistics results per read-back
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
