@@ -301,7 +301,7 @@ def batched_run(A, prob, frames: int, width: int, plain_value: float, mode: str 
     t0 = time.time()
     B = M.Batch(A, Y, budgets, rel_tol=1e-6, block_width=width, mode=mode)
     create_s = time.time() - t0
-    B.run(1)  # warm-up: graph capture, first launches
+    B.run(1)  # warm-up: first launches
     done0 = B.progress()["frame_iterations"]
     M.device_sync()
     t0 = time.perf_counter()
@@ -320,9 +320,9 @@ def batched_run(A, prob, frames: int, width: int, plain_value: float, mode: str 
                                     "mean": float(np.mean(its))},
            "early_stopped_frames": int(sum(1 for f in range(frames) if its[f] < budgets[f])),
            "generation_s": gen, "create_s": create_s,
-           "note": "the timed span starts after the first batched iteration (graph "
-                   "capture); create_s includes building the matrix's tiling and timing "
-                   "the block widths"}
+           "note": "the timed span starts after the first batched iteration; "
+                   "create_s includes building the matrix's tiling and timing the block "
+                   "widths"}
     if parity:
         from oracle import oracle as orc  # parity check only
         m = prob.matrix

@@ -334,7 +334,9 @@ typedef struct mlem_batch_options {
                        into the blocks that minimise the summed measured
                        time, single frames included                       */
   int use_graph;    /* 1: long runs without a stopping frame replay captured
-                       hipGraphs of several iterations; 0: direct launches  */
+                       hipGraphs of several iterations; 0: direct launches.
+                       With rel_tol > 0 a frame can stop after any
+                       iteration: always direct launches                    */
   int mode;         /* MLEM_MODE_FAST (default): blocks run through the
                        matrix's box tiling (16x16x4-voxel boxes whose slice
                        of a block, or whose voxel sums, stay in one

@@ -503,13 +503,6 @@ void collect_stats(mlem_recon* R, int first, int count) {
   }
 }
 
-// Captured iterations are replayed kGraphIterations at a time, in runs of at
-// least kGraphMin: a graph of one iteration (two kernels) costs 5-15 us more
-// per iteration than launching them (its launch waits for the one before: pet
-// 425 against 408 us, the 38,496-element matrix 21.9 against 13.8), one of 16
-// iterations 1.3 us less, and building it takes about 100 us.
-constexpr int kGraphIterations = 16, kGraphMin = 96;
-
 void drop_graph(mlem_recon* R) {
   if (R->exec) (void)hipGraphExecDestroy(R->exec);
   if (R->graph) (void)hipGraphDestroy(R->graph);

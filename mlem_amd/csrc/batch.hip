@@ -457,7 +457,6 @@ struct mlem_batch {
   std::vector<std::unique_ptr<RhsBlock>> blocks;
   std::vector<std::unique_ptr<RhsBlock>> spare;  // blocks kept for reuse by repacking
   float* final_x = nullptr;    // [F][cols] file order: images of finished frames
-  int32_t* y_file = nullptr;   // [F][rows] file order (kept for repacking)
   uint2* tiles_f = nullptr;
   uint2* tiles_b = nullptr;
   uint32_t nt_f = 0, nt_b = 0;
@@ -470,7 +469,6 @@ struct mlem_batch {
     if (graph) (void)hipGraphDestroy(graph);
     blocks.clear();
     dfree(final_x);
-    dfree(y_file);
     dfree(tiles_f);
     dfree(tiles_b);
     dfree(fpart);
@@ -657,9 +655,7 @@ void enqueue_iteration(mlem_batch* B, hipStream_t s) {
 }
 
 // n iterations. Blocks change whenever a frame stops, and a captured graph
-// with them (0.1-0.4 ms to build), so iterations are launched directly; runs
-// of at least kGraphMin are replayed kGraphIterations at a time.
-constexpr int kGraphIterations = 16, kGraphMin = 96;
+// with them (0.1-0.4 ms to build): only runs of at least kGraphMin are replayed.
 void enqueue_iterations(mlem_batch* B, int n, hipStream_t s) {
   int i = 0;
   if (B->use_graph) {
@@ -946,8 +942,12 @@ int mlem_batch_create(mlem_matrix* h, uint32_t frames, const int32_t* y, uint32_
     MLEM_HIP(hipMemcpyAsync(B->tiles_b, db.data(), sizeof(uint2) * db.size(),
                             hipMemcpyHostToDevice, m.stream));
     MLEM_HIP(hipMalloc(&B->final_x, 4ull * m.cols * frames));
-    MLEM_HIP(hipMalloc(&B->y_file, 4ull * m.rows * frames));
-    MLEM_HIP(hipMemcpyAsync(B->y_file, y, 4ull * m.rows * frames, hipMemcpyHostToDevice,
+    struct Counts {  // [F][rows] file order, until the blocks hold them
+      int32_t* p = nullptr;
+      ~Counts() { dfree(p); }
+    } y_file;
+    MLEM_HIP(hipMalloc(&y_file.p, 4ull * m.rows * frames));
+    MLEM_HIP(hipMemcpyAsync(y_file.p, y, 4ull * m.rows * frames, hipMemcpyHostToDevice,
                             m.stream));
     // x0 per frame: (float)(sum y / sum norm), initImage (seqcsr4mlem.cpp:52-66)
     std::vector<float> x0(frames);
@@ -960,7 +960,7 @@ int mlem_batch_create(mlem_matrix* h, uint32_t frames, const int32_t* y, uint32_
       MLEM_HIP(hipMalloc(&d.p, sizeof(CountSum) * frames));
       launch_fill(reinterpret_cast<float*>(d.p), 0.f, sizeof(CountSum) / 4 * (size_t)frames,
                   m.stream);
-      launch_count_sums(B->y_file, rows, frames, d.p, m.stream);
+      launch_count_sums(y_file.p, rows, frames, d.p, m.stream);
       MLEM_HIP(hipMemcpyAsync(sums.data(), d.p, sizeof(CountSum) * frames, hipMemcpyDeviceToHost,
                               m.stream));
       MLEM_HIP(hipStreamSynchronize(m.stream));
@@ -991,7 +991,7 @@ int mlem_batch_create(mlem_matrix* h, uint32_t frames, const int32_t* y, uint32_
       hipLaunchKernelGGL(k_lane_fill, dim3(blocks_for(m.cols)), dim3(kBlock), 0, m.stream, b.X,
                          b.W, l, x0[f], m.cols);
       hipLaunchKernelGGL(k_lane_y, dim3(blocks_for(m.rows)), dim3(kBlock), 0, m.stream, b.Y, b.W,
-                         l, B->y_file + (size_t)f * m.rows, m.rowold, m.rows);
+                         l, y_file.p + (size_t)f * m.rows, m.rowold, m.rows);
       ++l;
     }
     check_launch("batch setup");

@@ -398,7 +398,7 @@ namespace {
 // whatever stream they ran).
 //
 // What bounds it: the host link (52 GB/s). A packed part has 5.1 instead of 8
-// bytes per element where rows are lines of response in file order (2.4 % of the
+// bytes per element where rows are lines of response in file order (3 % of the
 // codes are escapes); 67.4M elements a pass: 10.3 -> 6.9 ms.
 template <class K>
 void stream_pass(const DevMatrix& m, bool csc, K&& kernel, hipStream_t s) {
