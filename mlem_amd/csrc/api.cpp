@@ -240,25 +240,25 @@ GroupLaunch named_launch(int kind, int param, const GroupLaunch& open) {
 // summed with direct gathers (EXACT: by one lane), so tiles hold the longest
 // segment where the largest ones can.
 // mlem_autotune measures the alternatives on the real matrix.
-GroupLaunch default_launch(uint64_t nnz, const std::vector<uint32_t>& ptr, const uint2* el,
-                           uint32_t dim, hipStream_t s) {
-  constexpr double kMoreLines = 250000.0;
+constexpr uint64_t kSmallNnz = 2500000, kMidNnz = 20000000, kMoreLines = 250000;
+GroupLaunch default_launch(uint64_t nnz, const std::vector<uint32_t>& ptr,
+                           const std::array<double, 3>& lines) {
   GroupLaunch g = make_launch(kDictWide, 32);  // the same FAST sums with every tile size
-  if (nnz > 20000000 || nnz == 0 || !el) return g;
+  if (nnz > kMidNnz || nnz == 0) return g;
   uint32_t longest = 0;
-  double squares = 0.0;
+  uint64_t squares = 0;
   for (size_t i = 0; i + 1 < ptr.size(); ++i) {
     const uint32_t n = ptr[i + 1] - ptr[i];
     longest = std::max(longest, n);
-    squares += (double)n * n;
+    squares += (uint64_t)n * n;
   }
-  const double length = squares / (double)nnz;  // of an element's segment, on average
-  if (longest + 3 > 512 * 16 || (nnz > 2500000 && length > 512 * 16 / 5)) return g;
-  const std::array<double, 3> lines = tile_lines(ptr, el, dim, s);
-  if (lines[1] - lines[0] > kMoreLines) return g;
+  const double length = (double)squares / (double)nnz;  // of an element's segment, on average
+  if (longest + 3 > 512 * 16 || (nnz > kSmallNnz && length > 512 * 16 / 5) ||
+      lines[1] - lines[0] > (double)kMoreLines)
+    return g;
   g = make_launch(kDictWide, 16);
-  if (nnz <= 2500000 && longest + 3 <= 256 * 8 && length <= 256 * 8 / 5 &&
-      lines[2] - lines[1] <= kMoreLines)
+  if (nnz <= kSmallNnz && longest + 3 <= 256 * 8 && length <= 256 * 8 / 5 &&
+      lines[2] - lines[1] <= (double)kMoreLines)
     g = make_launch(kDict, 8);
   g.nested = true;
   return g;
@@ -393,8 +393,15 @@ void finish_open(mlem_matrix* h, unsigned flags) {
 
   const double avgRow = m.rows ? (double)m.nnz / m.rows : 1.0;
   download_pointers(m, m.stream);
-  m.fwd = m.fwd_open = default_launch(m.nnz, m.h_rowptr, m.csr, m.cols, m.stream);
-  m.bwd = m.bwd_open = default_launch(m.nnz, m.h_colptr, m.csc, m.rows, m.stream);
+  GatherSide f{&m.h_rowptr, m.csr, m.cols}, b{&m.h_colptr, m.csc, m.rows};
+  if (m.nnz > kMoreLines && m.nnz <= kMidNnz) {  // (no tiles touch more lines than elements)
+    if (m.csc)
+      tile_lines({&f, &b}, m.stream);
+    else
+      tile_lines({&f}, m.stream);
+  }
+  m.fwd = m.fwd_open = default_launch(m.nnz, m.h_rowptr, f.lines);
+  m.bwd = m.bwd_open = default_launch(m.nnz, m.h_colptr, b.lines);
   m.scatter = make_launch(kGroups, lanes_for(avgRow));
   prepare_tiles(m, m.stream);
   if (env_int("MLEM_AUTOTUNE", 0) > 0) autotune(m);

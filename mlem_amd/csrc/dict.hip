@@ -18,7 +18,7 @@
 // pass per slab that holds an element: up to one per element where the indices
 // spread far), a bitonic sort of 8-byte keys in LDS 43 / 110 / 222 and 8.9 / 27 / 89.
 #include <algorithm>
-#include <array>
+#include <initializer_list>
 #include <vector>
 
 #include "internal.hpp"
@@ -388,53 +388,68 @@ std::vector<uint32_t> partition_tiles(const std::vector<uint32_t>& ptr, uint32_t
   return tiles;
 }
 
-std::array<double, 3> tile_lines(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim,
-                                 hipStream_t s) {
+void tile_lines(std::initializer_list<GatherSide*> sides, hipStream_t s) {
   constexpr uint32_t kSample = 64, T[3] = {16384, 8192, 2048}, kSeg[3] = {512, 512, 256};
-  const uint32_t n = (uint32_t)ptr.size() - 1;
   // the tiles of every size in the sampled large ones, one after the other: a
   // range of elements from each entry to the next, those in which `size` is set
   std::vector<uint2> range;
   std::vector<int> size;
-  uint64_t covered = 0;
-  for (uint32_t i = 0, s0 = 0, s1 = 0; i < kSample && s1 < n; ++i) {
-    s0 = std::max(s1, (uint32_t)((uint64_t)n * i / kSample));
-    s1 = s0 + 1;
-    while (s1 < n && s1 - s0 < kSeg[0] && ptr[s1 + 1] - ptr[s0] <= T[0]) ++s1;
-    covered += ptr[s1] - ptr[s0];
-    for (int k = 0; k < 3; ++k) {
-      cut_nested(ptr, s0, s1, T[k], kSeg[k], [&](uint32_t b, uint32_t, uint32_t) {
-        range.push_back(make_uint2(b, ptr[b]));
-        size.push_back(k);
-      });
-      range.push_back(make_uint2(s1, ptr[s1]));
-      size.push_back(-1);
+  std::vector<size_t> end;  // of each side's entries
+  std::vector<uint64_t> covered;
+  for (GatherSide* g : sides) {
+    const std::vector<uint32_t>& ptr = *g->ptr;
+    const uint32_t n = (uint32_t)ptr.size() - 1;
+    covered.push_back(0);
+    for (uint32_t i = 0, s0 = 0, s1 = 0; i < kSample && s1 < n; ++i) {
+      s0 = std::max(s1, (uint32_t)((uint64_t)n * i / kSample));
+      s1 = s0 + 1;
+      while (s1 < n && s1 - s0 < kSeg[0] && ptr[s1 + 1] - ptr[s0] <= T[0]) ++s1;
+      covered.back() += ptr[s1] - ptr[s0];
+      for (int k = 0; k < 3; ++k) {
+        cut_nested(ptr, s0, s1, T[k], kSeg[k], [&](uint32_t b, uint32_t, uint32_t) {
+          range.push_back(make_uint2(b, ptr[b]));
+          size.push_back(k);
+        });
+        range.push_back(make_uint2(s1, ptr[s1]));
+        size.push_back(-1);
+      }
     }
+    end.push_back(range.size());
   }
-  std::array<double, 3> lines{0.0, 0.0, 0.0};
-  if (range.size() < 2 || covered == 0) return lines;
+  if (range.empty()) return;
   struct Buf {
     void* p = nullptr;
     ~Buf() {
       if (p) (void)hipFree(p);
     }
   } buf;
-  std::vector<uint2> counts(range.size() - 1);
+  std::vector<uint2> counts(range.size());
   MLEM_HIP(hipMalloc(&buf.p, 2 * sizeof(uint2) * range.size()));
   uint2 *d_range = static_cast<uint2*>(buf.p), *d_counts = d_range + range.size();
   MLEM_HIP(hipMemcpyAsync(d_range, range.data(), sizeof(uint2) * range.size(),
                           hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL((k_dict_rank<16, kF32>), dim3((unsigned)counts.size()), dim3(kBuild), 0, s, el,
-                     (const uint2*)d_range, (const uint4*)nullptr, 0u, page_bits_for(dim), d_counts,
-                     (uint32_t*)nullptr, (void*)nullptr, (uint16_t*)nullptr);
+  size_t at = 0, i = 0;
+  for (GatherSide* g : sides) {
+    const size_t n = end[i++] - at;
+    if (n > 1)
+      hipLaunchKernelGGL((k_dict_rank<16, kF32>), dim3((unsigned)n - 1), dim3(kBuild), 0, s, g->el,
+                         (const uint2*)(d_range + at), (const uint4*)nullptr, 0u,
+                         page_bits_for(g->dim), d_counts + at, (uint32_t*)nullptr, (void*)nullptr,
+                         (uint16_t*)nullptr);
+    at += n;
+  }
   check_launch("tile sample launch");
   MLEM_HIP(hipMemcpyAsync(counts.data(), d_counts, sizeof(uint2) * counts.size(),
                           hipMemcpyDeviceToHost, s));
   MLEM_HIP(hipStreamSynchronize(s));
-  for (size_t i = 0; i < counts.size(); ++i)
-    if (size[i] >= 0) lines[(size_t)size[i]] += counts[i].y;
-  for (double& l : lines) l *= (double)ptr[n] / (double)covered;
-  return lines;
+  at = i = 0;
+  for (GatherSide* g : sides) {
+    for (; at < end[i]; ++at)
+      if (size[at] >= 0) g->lines[(size_t)size[at]] += counts[at].y;
+    if (covered[i])
+      for (double& l : g->lines) l *= (double)g->ptr->back() / (double)covered[i];
+    ++i;
+  }
 }
 
 void ensure_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, int nb, int ept,

@@ -317,10 +317,16 @@ std::vector<uint32_t> partition_tiles(const std::vector<uint32_t>& ptr, uint32_t
 void ensure_dict(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim, int nb, int ept,
                  bool nested, int vk, DictFormat& D, hipStream_t s);
 // Lines (32 neighbouring entries of the gathered vector) that the dictionary tiles
-// of 16384, 8192 and 2048 elements touch in all, the smaller ones nested in the
-// larger: estimated from up to 64 of the large tiles, exact if there are no more.
-std::array<double, 3> tile_lines(const std::vector<uint32_t>& ptr, const uint2* el, uint32_t dim,
-                                 hipStream_t s);
+// of 16384, 8192 and 2048 elements of a projection touch in all, the smaller ones
+// nested in the larger: estimated from up to 64 of the large tiles, exact if there
+// are no more.
+struct GatherSide {
+  const std::vector<uint32_t>* ptr;  // first element of each segment, and the end
+  const uint2* el;                   // elements, indices below dim
+  uint32_t dim;
+  std::array<double, 3> lines{0.0, 0.0, 0.0};
+};
+void tile_lines(std::initializer_list<GatherSide*> sides, hipStream_t s);
 // Release a dictionary format's device memory.
 void free_dict(DictFormat& d);
 // Forward projection. ratio: out = (f != 0) ? y/f : 0, else out = f.
