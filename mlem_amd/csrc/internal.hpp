@@ -130,8 +130,7 @@ struct GroupLaunch {
 // elements with code kPackEscape, each padded to 16 bytes: the column of an
 // element is the column before it in the chunk (0 before the first) plus, modulo
 // 2^32, the step of its code. A chunk that would not become smaller holds the
-// 8-byte records (steps = kPackRaw). Groups of chunks that were packed by
-// different threads keep the places of their first elements.
+// 8-byte records (steps = kPackRaw).
 //
 // Why from 2^20 elements on: below, a block's kernels take longer than the copy of
 // its 8-byte records (8 MB: 168 us against 160; 4 MB: 145 against 80), and
@@ -154,10 +153,7 @@ struct StreamBlock {
   uint32_t row0 = 0, rows = 0;  // first row, rows
   uint64_t nnz = 0;
   uint64_t csr_off = 0, csr_bytes = 0;  // parts within the host buffer
-  struct Range {
-    uint64_t at, bytes;
-  };
-  std::vector<Range> packed;  // ranges of the packed CSR part that are copied; none: not packed
+  uint64_t packed_bytes = 0;            // of the packed CSR part; 0: not packed
   uint64_t csc_off = 0, csc_bytes = 0;
   char* resident = nullptr;  // device copy of both parts (CSR, then CSC), or none
 };

@@ -322,47 +322,64 @@ StreamedMatrix* build_streamed(uint32_t rows, uint32_t cols, uint64_t nnz,
   on_threads(nthreads, work);
   check();
 
-  // Pack: a matrix of few blocks has each cut into groups of chunks, so that more
-  // threads have some (about 1 ns an element on one thread: 67M elements in one
-  // block 75 ms, opened in 690). The groups keep their places, so every one is a
-  // copy of its own, and those cost about 9 us each: at most four.
+  // Pack: a matrix of few blocks has each cut into groups of chunks, so that every
+  // thread has some (about 1 ns an element on one thread: 67M elements in one block
+  // 75 ms, opened in 690); then the groups of a block are moved together, so that it
+  // crosses the link in one copy (each further one costs about 9 us a pass).
   struct Group {
     size_t block;
     uint64_t c0, c1;
+    char *begin, *end;
   };
   std::vector<Group> groups;
+  std::vector<size_t> first_group;  // of each packed block, and the end
+  auto front_of = [&](const StreamBlock& B) {
+    return S->host + B.csr_off + align16(4ull * ((uint64_t)B.rows + 1));
+  };
   for (size_t b = 0; b < S->blocks.size(); ++b) {
-    StreamBlock& B = S->blocks[b];
+    const StreamBlock& B = S->blocks[b];
     if (!steps[b].pays) continue;
     const uint64_t n = pack_chunks_of(B.nnz);
     const uint64_t g = std::max<uint64_t>(
-        1, std::min<uint64_t>({hw / S->blocks.size(), B.nnz / kPackMin, 4}));
-    B.packed.resize(g);
-    for (uint64_t i = 0; i < g; ++i) groups.push_back(Group{b, n * i / g, n * (i + 1) / g});
-    char* front = S->host + B.csr_off + align16(4ull * ((uint64_t)B.rows + 1));
-    std::memcpy(front + sizeof(PackHead) * n, steps[b].step, sizeof(steps[b].step));
+        1, std::min<uint64_t>(hw / S->blocks.size(), B.nnz / kPackMin));
+    std::memcpy(front_of(B) + sizeof(PackHead) * n, steps[b].step, sizeof(steps[b].step));
+    first_group.push_back(groups.size());
+    for (uint64_t i = 0; i < g; ++i)
+      groups.push_back(Group{b, n * i / g, n * (i + 1) / g, nullptr, nullptr});
   }
-  std::atomic<size_t> next_group{0};
+  first_group.push_back(groups.size());
+  const size_t npacked = first_group.size() - 1;
+  std::atomic<size_t> next_group{0}, next_block{0};
   auto pack = [&](unsigned tid) {
     try {
       for (size_t i; (i = next_group++) < groups.size();) {
-        const Group& G = groups[i];
-        StreamBlock& B = S->blocks[G.block];
-        char* csr = S->host + B.csr_off;
-        char* front = csr + align16(4ull * ((uint64_t)B.rows + 1));
-        char* begin = G.c0 ? front + pack_front(B.nnz) + 8ull * kPackChunk * G.c0 : csr;
-        char* end = pack_chunks(front, B.nnz, G.c0, G.c1, steps[G.block]);
-        size_t at = 0;  // of this group among its block's
-        while (i > at && groups[i - at - 1].block == G.block) ++at;
-        B.packed[at] = {(uint64_t)(begin - csr), (uint64_t)(end - begin)};
+        Group& G = groups[i];
+        const StreamBlock& B = S->blocks[G.block];
+        G.begin = front_of(B) + pack_front(B.nnz) + 8ull * kPackChunk * G.c0;
+        G.end = pack_chunks(front_of(B), B.nnz, G.c0, G.c1, steps[G.block]);
       }
     } catch (const std::exception& e) {
       errors[tid] = e.what();
     }
   };
-  if (!groups.empty()) {
+  auto join = [&](unsigned) {
+    for (size_t k; (k = next_block++) < npacked;) {
+      StreamBlock& B = S->blocks[groups[first_group[k]].block];
+      PackHead* heads = reinterpret_cast<PackHead*>(front_of(B));
+      char* end = groups[first_group[k]].end;
+      for (size_t i = first_group[k] + 1; i < first_group[k + 1]; ++i) {
+        const Group& G = groups[i];
+        for (uint64_t c = G.c0; c < G.c1; ++c) heads[c].at -= (uint32_t)((G.begin - end) / 16);
+        std::memmove(end, G.begin, (size_t)(G.end - G.begin));
+        end += G.end - G.begin;
+      }
+      B.packed_bytes = (uint64_t)(end - (S->host + B.csr_off));
+    }
+  };
+  if (npacked) {
     on_threads((unsigned)std::min<size_t>(groups.size(), hw), pack);
     check();
+    on_threads((unsigned)std::min<size_t>(npacked, hw), join);
   } else if (S->expand) {  // nothing to unpack
     MLEM_HIP(hipFree(S->expand));
     S->expand = nullptr;
@@ -414,16 +431,11 @@ void stream_pass(const DevMatrix& m, bool csc, K&& kernel, hipStream_t s) {
       continue;
     }
     const int i = (int)(n_streamed++ & 1);
-    const bool packed = !csc && !B.packed.empty();
+    const bool packed = !csc && B.packed_bytes;
+    const uint64_t off = csc ? B.csc_off : B.csr_off;
+    const uint64_t n = csc ? B.csc_bytes : packed ? B.packed_bytes : B.csr_bytes;
     MLEM_HIP(hipStreamWaitEvent(S.copy, S.freed[i], 0));
-    if (packed) {
-      for (const StreamBlock::Range& g : B.packed)
-        MLEM_HIP(hipMemcpyAsync(S.dev[i] + g.at, S.host + B.csr_off + g.at, g.bytes,
-                                hipMemcpyHostToDevice, S.copy));
-    } else {
-      MLEM_HIP(hipMemcpyAsync(S.dev[i], S.host + (csc ? B.csc_off : B.csr_off),
-                              csc ? B.csc_bytes : B.csr_bytes, hipMemcpyHostToDevice, S.copy));
-    }
+    MLEM_HIP(hipMemcpyAsync(S.dev[i], S.host + off, n, hipMemcpyHostToDevice, S.copy));
     MLEM_HIP(hipEventRecord(S.copied[i], S.copy));
     MLEM_HIP(hipStreamWaitEvent(s, S.copied[i], 0));
     const uint2* el = reinterpret_cast<const uint2*>(S.dev[i] + pointers);
