@@ -457,6 +457,9 @@ struct mlem_batch {
   std::vector<std::unique_ptr<RhsBlock>> blocks;
   std::vector<std::unique_ptr<RhsBlock>> spare;  // blocks kept for reuse by repacking
   float* final_x = nullptr;    // [F][cols] file order: images of finished frames
+  // [F][rows] file order, read at creation only (freed with the batch: freeing
+  // it at creation made 13 EXACT frames of 20 iterations take 8.7 instead of 8.2 ms)
+  int32_t* y_file = nullptr;
   uint2* tiles_f = nullptr;
   uint2* tiles_b = nullptr;
   uint32_t nt_f = 0, nt_b = 0;
@@ -469,6 +472,7 @@ struct mlem_batch {
     if (graph) (void)hipGraphDestroy(graph);
     blocks.clear();
     dfree(final_x);
+    dfree(y_file);
     dfree(tiles_f);
     dfree(tiles_b);
     dfree(fpart);
@@ -942,12 +946,8 @@ int mlem_batch_create(mlem_matrix* h, uint32_t frames, const int32_t* y, uint32_
     MLEM_HIP(hipMemcpyAsync(B->tiles_b, db.data(), sizeof(uint2) * db.size(),
                             hipMemcpyHostToDevice, m.stream));
     MLEM_HIP(hipMalloc(&B->final_x, 4ull * m.cols * frames));
-    struct Counts {  // [F][rows] file order, until the blocks hold them
-      int32_t* p = nullptr;
-      ~Counts() { dfree(p); }
-    } y_file;
-    MLEM_HIP(hipMalloc(&y_file.p, 4ull * m.rows * frames));
-    MLEM_HIP(hipMemcpyAsync(y_file.p, y, 4ull * m.rows * frames, hipMemcpyHostToDevice,
+    MLEM_HIP(hipMalloc(&B->y_file, 4ull * m.rows * frames));
+    MLEM_HIP(hipMemcpyAsync(B->y_file, y, 4ull * m.rows * frames, hipMemcpyHostToDevice,
                             m.stream));
     // x0 per frame: (float)(sum y / sum norm), initImage (seqcsr4mlem.cpp:52-66)
     std::vector<float> x0(frames);
@@ -960,7 +960,7 @@ int mlem_batch_create(mlem_matrix* h, uint32_t frames, const int32_t* y, uint32_
       MLEM_HIP(hipMalloc(&d.p, sizeof(CountSum) * frames));
       launch_fill(reinterpret_cast<float*>(d.p), 0.f, sizeof(CountSum) / 4 * (size_t)frames,
                   m.stream);
-      launch_count_sums(y_file.p, rows, frames, d.p, m.stream);
+      launch_count_sums(B->y_file, rows, frames, d.p, m.stream);
       MLEM_HIP(hipMemcpyAsync(sums.data(), d.p, sizeof(CountSum) * frames, hipMemcpyDeviceToHost,
                               m.stream));
       MLEM_HIP(hipStreamSynchronize(m.stream));
@@ -991,7 +991,7 @@ int mlem_batch_create(mlem_matrix* h, uint32_t frames, const int32_t* y, uint32_
       hipLaunchKernelGGL(k_lane_fill, dim3(blocks_for(m.cols)), dim3(kBlock), 0, m.stream, b.X,
                          b.W, l, x0[f], m.cols);
       hipLaunchKernelGGL(k_lane_y, dim3(blocks_for(m.rows)), dim3(kBlock), 0, m.stream, b.Y, b.W,
-                         l, y_file.p + (size_t)f * m.rows, m.rowold, m.rows);
+                         l, B->y_file + (size_t)f * m.rows, m.rowold, m.rows);
       ++l;
     }
     check_launch("batch setup");
